@@ -55,9 +55,13 @@ void memory_stats(long *cur, long *peak, long *n);
 // kernel that uses the scratch is enqueued, so that another host thread cannot enqueue
 // work that reuses it in between (kernels on one stream run in order).
 void *stream_scratch(hipStream_t s, size_t bytes, std::unique_lock<std::mutex> &lk, CError *err);
+// Scratch blocks above this size go back to the pool after the call that needed them (see
+// stream_scratch_trim): the pool's cache can hand them out again or, when hipMalloc fails,
+// return them to the driver, which it cannot do with a block a stream keeps.
+constexpr size_t kScratchRetainBytes = (size_t)512 << 20;
 // Called with lk still held, after the kernels that use the scratch are enqueued: a block
-// above 256 MiB is released (stream-ordered) instead of being kept for the stream's next
-// call, so one large call does not pin it for the life of the process.
+// above kScratchRetainBytes is released (stream-ordered) instead of being kept for the stream's
+// next call, so one large call does not pin it for the life of the process.
 void stream_scratch_trim(hipStream_t s, std::unique_lock<std::mutex> &lk);
 
 // ---------------------------------------------------------------- host <-> device

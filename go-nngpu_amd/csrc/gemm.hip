@@ -25,170 +25,13 @@
 //  * a grouped, XCD-aware tile order: hardware dispatches workgroup w to XCD w % 8,
 //    so w is remapped to give each XCD a contiguous band of tiles that share A/B
 //    panels in that XCD's L2.
-#include "act.h"
-#include "common.h"
-#include "ring_plan.h"
+#include "gemm_split.h"
+#include "gemm_tile.h"
+
+#include <atomic>
 
 namespace gn {
 namespace {
-
-typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
-typedef float float4_t __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
-typedef __fp16 trh4_t __attribute__((__vector_size__(4 * sizeof(__fp16))));
-typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
-
-#define LDS_AS __attribute__((address_space(3)))
-
-struct GemmParams {
-  const void *A;
-  const void *B;
-  float *C;
-  const float *bias;
-  long M, N, K;
-  long lda, ldb, ldc;
-  long strideA, strideB, strideC;
-  float alpha, beta, act_alpha;
-  int act;
-  int tiles_m, tiles_n;
-  int group_m;  // tile rows per raster group (tile_coords); 0 selects the default of 4
-};
-
-// ------------------------------------------------------------------ epilogue
-// Workgroup barrier that orders LDS accesses only (s_waitcnt lgkmcnt(0); s_barrier).
-// __syncthreads() also waits for vmcnt(0), i.e. for every global store the wave has
-// issued to complete, which between the epilogue's passes serialised each pass behind
-// the previous pass's C writes.
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
-template <int V>
-struct ActCode {
-  static constexpr int value = V;
-};
-constexpr int kActRuntime = -1000;  // ActCode value: apply p.act, decided per element
-
-// Writes a workgroup's BM x BN accumulator tile to C in row order. Pass f stages MFMA
-// block-row f of every wave (WM x 16 tile rows, all BN columns) in LDS at `stg` (pitch
-// BN + 4 floats: the 4 row groups of one ds_write_b32 fall on distinct banks), then the
-// workgroup stores those rows as 16-byte vectors with consecutive lanes along a row, so
-// each store instruction writes long contiguous row segments (one whole 1 KiB row at
-// BN = 256). All CUs write their tiles at about the same time; when each wave stored
-// only its own 256-byte row pieces (rows 32 KiB apart), the writes drained so slowly
-// that the 8192^3 GEMM took 11% longer (4096^3: 17%). Each thread owns one column quad
-// for the whole epilogue, so its bias values are loaded once, before the first pass: a
-// load inside the passes would wait for all earlier stores (vmcnt counts stores too).
-// The passes are separated by LDS-only barriers, so the stores of one pass drain while
-// the next is staged. alpha, beta*C, bias and the activation are applied on the way;
-// scalar stores at ragged edges or when ldc / C do not allow aligned 16-byte stores.
-// The pass loop is unrolled so every accumulator index is static (a runtime index would
-// move the accumulators to scratch memory). stage(f) writes the wave's rows of pass f (wave
-// tile rows 16 f .. 16 f + 15) into stg at rows wm * 16 + 0..15, pitch BN + 4, columns
-// wn * (BN / WN) + 0..BN / WN - 1.
-template <int BM, int BN, int WM, int WN, typename Stage>
-__device__ __forceinline__ void store_tile_passes(const GemmParams &p, long m0, long n0, long z, float *stg,
-                                                  Stage &&stage) {
-  constexpr int WTM = BM / WM, FM = WTM / 16;
-  constexpr int LP = BN + 4, CPR = BN / 4, NTH = WM * WN * 64;
-  constexpr int ROWS = WM * 16;       // tile rows staged per pass
-  constexpr int RPS = NTH / CPR;      // rows one sweep of the workgroup's threads covers
-  constexpr int SWEEPS = (ROWS + RPS - 1) / RPS;
-  static_assert(BN % 4 == 0 && CPR <= NTH, "row vectors");
-  const int c4 = threadIdx.x % CPR, r0 = threadIdx.x / CPR;  // threads with r0 >= RPS only stage
-  const long col = n0 + 4 * c4;
-  float *C = p.C + z * p.strideC;
-  const bool vec = (p.ldc % 4 == 0) && (((uintptr_t)C & 15) == 0) && col + 3 < p.N;
-  float bv[4];
-#pragma unroll
-  for (int e = 0; e < 4; ++e) bv[e] = (p.bias && col + e < p.N) ? p.bias[col + e] : 0.0f;
-#pragma unroll
-  for (int f = 0; f < FM; ++f) {
-    lds_barrier();  // the previous pass (or the main loop) is done with stg
-    stage(f);
-    lds_barrier();
-    // The common activations get their own copy of the row sweep with the code fixed at
-    // compile time: the generic one inlines every case of apply_act for every element,
-    // and that long branchy code cost 3.5 us per launch at 512 x 11008 x 512 (ReLU).
-    auto sweep = [&](auto act_c) {
-      constexpr int ACT = decltype(act_c)::value;
-      const int act = ACT == kActRuntime ? p.act : ACT;
-      // a runtime loop: unrolling it as well made the pass loop too large to unroll
-      // fully (the 256 x 256 kernels then kept the accumulators in scratch memory)
-#pragma unroll 1
-      for (int s = 0; s < SWEEPS; ++s) {
-        const int t = r0 + s * RPS;
-        if (r0 >= RPS || t >= ROWS) continue;
-        const long row = m0 + (t / 16) * WTM + f * 16 + (t % 16);
-        if (row >= p.M) continue;
-        const float4_t v = *reinterpret_cast<const float4_t *>(stg + t * LP + 4 * c4);
-        float *dst = C + row * p.ldc + col;
-        if (vec) {
-          float4_t o;
-          const float4_t old =
-              p.beta != 0.0f ? *reinterpret_cast<const float4_t *>(dst) : float4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int e = 0; e < 4; ++e) o[e] = apply_act(act, p.alpha * v[e] + p.beta * old[e] + bv[e], p.act_alpha);
-          __builtin_nontemporal_store(o, reinterpret_cast<float4_t *>(dst));  // C is not re-read: keep L2 for A/B
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            if (col + e < p.N) {
-              float x = p.alpha * v[e];
-              if (p.beta != 0.0f) x += p.beta * dst[e];
-              dst[e] = apply_act(act, x + bv[e], p.act_alpha);
-            }
-          }
-        }
-      }
-    };
-    switch (p.act) {
-      case -1: sweep(ActCode<-1>{}); break;
-      case 0: sweep(ActCode<0>{}); break;
-      case 7: sweep(ActCode<7>{}); break;
-      default: sweep(ActCode<kActRuntime>{}); break;
-    }
-  }
-}
-
-// store_tile_passes for 16 x 16 MFMA accumulators: lane (c, g) of block (f, j) holds rows
-// 4 g + 0..3 of column c.
-template <int BM, int BN, int WM, int WN>
-__device__ __forceinline__ void store_tile_rows(const GemmParams &p, long m0, long n0, long z, float *stg,
-                                                const float4_t (&acc)[BM / WM / 16][BN / WN / 16]) {
-  constexpr int WTN = BN / WN, FN = WTN / 16, LP = BN + 4;
-  const int wave = threadIdx.x >> 6, wm = wave / WN, wn = wave % WN, lane = threadIdx.x & 63;
-  const int c = lane & 15, g = lane >> 4;
-  store_tile_passes<BM, BN, WM, WN>(p, m0, n0, z, stg, [&](int f) {
-#pragma unroll
-    for (int j = 0; j < FN; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) stg[(wm * 16 + 4 * g + r) * LP + wn * WTN + 16 * j + c] = acc[f][j][r];
-  });
-}
-
-// Grouped + XCD-aware mapping of the linear workgroup id to a (tile_m, tile_n) pair.
-__device__ __forceinline__ void tile_coords(const GemmParams &p, int &tm, int &tn) {
-  // Workgroup w runs on XCD w % 8; give XCD x the contiguous tile range
-  // [x*base + min(x, rem), ...) of base (+1 for the first rem XCDs) tiles.
-  const int total = p.tiles_m * p.tiles_n;
-  int w = blockIdx.x;
-  {
-    const int base = total >> 3, rem = total & 7, x = w & 7;
-    w = x * base + min(x, rem) + (w >> 3);
-  }
-  const int GROUP_M = p.group_m > 0 ? p.group_m : 4;
-  const int in_group = GROUP_M * p.tiles_n;
-  const int group = w / in_group;
-  const int first_m = group * GROUP_M;
-  const int gsize = min(p.tiles_m - first_m, GROUP_M);
-  const int r = w - group * in_group;
-  tm = first_m + r % gsize;
-  tn = r / gsize;
-}
 
 // ------------------------------------------------------------------ tile loads
 // A tile of R rows x CC contiguous elements is moved global -> registers -> LDS in
@@ -387,7 +230,9 @@ __global__ void __launch_bounds__(WM * WN * 64) gemm_f16_kernel(GemmParams p) {
 //    16-byte fragment reads (25 M conflict cycles per operand at 4096^3), so both tiles
 //    are stored transposed (four 4-byte writes, conflict-free for these loaders) and read
 //    as M/N-contiguous ones: 4096^3 NT 1045 -> 1020 us; NN, TN and TT do not gain.
-template <int BM, int BN, int BK, int WM, int WN, bool TA, bool TB, bool VEC>
+// GATED: stands behind a split product (GemmParams::gate); a template argument because the
+// gate's load, ahead of the other arguments', cost the 12 us batched products half a microsecond.
+template <int BM, int BN, int BK, int WM, int WN, bool TA, bool TB, bool VEC, bool GATED>
 __global__ void __launch_bounds__(WM * WN * 64) gemm_f32_kernel(GemmParams p) {
   constexpr int NT = WM * WN * 64;
   constexpr int WTM = BM / WM, WTN = BN / WN;
@@ -400,6 +245,7 @@ __global__ void __launch_bounds__(WM * WN * 64) gemm_f32_kernel(GemmParams p) {
   constexpr int A_ELEMS = MA ? BK * PA : BM * PA;
   constexpr int B_ELEMS = MB ? BK * PB : BN * PB;
   __shared__ __attribute__((aligned(16))) float smem[2 * (A_ELEMS + B_ELEMS)];
+  if (GATED && !fp32_needed(p)) return;
 
   int tm, tn;
   tile_coords(p, tm, tn);
@@ -663,61 +509,6 @@ __global__ void __launch_bounds__(KW * 64) gemm_small_kernel(GemmParams p) {
 // The DMA is issued from inline assembly so the compiler does not track these LDS
 // writes (it would otherwise wait for every outstanding load before each LDS read);
 // the kernel orders them itself with s_waitcnt vmcnt and the barriers.
-typedef int i32x4_t __attribute__((ext_vector_type(4)));
-
-struct BufRsrc {
-  i32x4_t r;
-};
-
-// Raw buffer descriptor: 48-bit base, stride 0, num_records ring::kNumRecords (offsets at
-// or beyond it read as zero), gfx9 dword3.
-__device__ __forceinline__ BufRsrc make_rsrc(const void *base) {
-  const unsigned long long b = (unsigned long long)base;
-  BufRsrc s;
-  s.r.x = __builtin_amdgcn_readfirstlane((int)(b & 0xffffffffu));
-  s.r.y = __builtin_amdgcn_readfirstlane((int)(b >> 32) & 0xffff);
-  s.r.z = (int)ring::kNumRecords;
-  s.r.w = 0x00020000;
-  return s;
-}
-
-__device__ __forceinline__ void rsrc_advance(BufRsrc &s, long bytes) {
-  unsigned long long b =
-      ((unsigned long long)(unsigned)s.r.x) | ((unsigned long long)(unsigned)(s.r.y & 0xffff) << 32);
-  b += (unsigned long long)bytes;
-  s.r.x = __builtin_amdgcn_readfirstlane((int)(b & 0xffffffffu));
-  s.r.y = __builtin_amdgcn_readfirstlane((int)(b >> 32) & 0xffff);
-}
-
-// 16 bytes per lane from the buffer at voff into LDS at lds + 16 * lane (lds is
-// wave-uniform). M0 is saved and restored around the load.
-__device__ __forceinline__ void dma16(const BufRsrc &s, unsigned voff, unsigned lds) {
-  int saved;
-  asm volatile(
-      "s_mov_b32 %0, m0\n\t"
-      "s_mov_b32 m0, %3\n\t"
-      "buffer_load_dwordx4 %1, %2, 0 offen lds\n\t"
-      "s_mov_b32 m0, %0"
-      : "=&s"(saved)
-      : "v"(voff), "s"(s.r), "s"(lds)
-      : "memory");
-}
-
-using ring::hsw;
-using ring::kc8_octet;
-using ring::kc8_slot;
-using ring::kOutOfRange;
-using ring::msw32;
-
-// s_waitcnt immediate that waits for vmcnt <= n only (vmcnt[3:0] in bits 3:0 and
-// vmcnt[5:4] in bits 15:14; expcnt and lgkmcnt at their maxima).
-constexpr int vmcnt_imm(int n) { return (n & 0xF) | ((n >> 4) << 14) | (0x7 << 4) | (0xF << 8); }
-
-__device__ __forceinline__ unsigned lds_offset(const void *p) {
-  return (unsigned)(unsigned long)(const LDS_AS void *)p;
-}
-
-
 // K-contiguous tiles: a 1 KiB DMA chunk holds rows 8c..8c+7 with the 64 k of a K-tile
 // pair (128 bytes) each. Lane L copies 16 bytes of row 8c + (L >> 3), so each lane
 // octet reads one whole 128-byte line: half the L1 requests of 16 rows x 64 bytes per
@@ -727,19 +518,6 @@ __device__ __forceinline__ unsigned lds_offset(const void *p) {
 // in slot 8 (r & 7) + (o ^ ((r >> 1) & 7)), and the 16 rows an MFMA fragment read
 // touches (two chunks, fixed o) land on 16 distinct 16-byte bank groups (ring::kc8_slot,
 // ring::kc8_octet).
-
-// A scheduling region of NM MFMAs and NR LDS reads, interleaved 1:1 (then the rest).
-template <int NM, int NR>
-__device__ __forceinline__ void sched_interleave() {
-  constexpr int NP = NR < NM ? NR : NM;
-#pragma unroll
-  for (int g = 0; g < NP; ++g) {
-    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-  }
-  if constexpr (NM > NP) __builtin_amdgcn_sched_group_barrier(0x008, NM - NP, 0);
-  if constexpr (NR > NP) __builtin_amdgcn_sched_group_barrier(0x100, NR - NP, 0);
-}
 
 // The copy side of the fp16 ring for one output tile: each wave's share of a K-tile pair's
 // 1 KiB DMA chunks into a ring slot. For a K-contiguous operand chunk c of a pair holds rows
@@ -1402,12 +1180,13 @@ __device__ __forceinline__ void ring_mainloop_f32(const GemmParams &p, long m0, 
   __syncthreads();
 }
 
-template <int BM, int BN, int WM, int WN, bool TA, bool TB, int WPE, int NS>
+template <int BM, int BN, int WM, int WN, bool TA, bool TB, int WPE, int NS, bool GATED>
 __global__ void __launch_bounds__(WM * WN * 64) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
 gemm_f32_ring_kernel(GemmParams p) {
   constexpr int FM = BM / WM / 16, FN = BN / WN / 16;
   constexpr int RING = NS * 2 * (BM + BN) * 16 * 4;  // NS slots of two K-tiles of A and B
   __shared__ __attribute__((aligned(1024))) char smem[RING];
+  if (GATED && !fp32_needed(p)) return;
   int tm, tn;
   tile_coords(p, tm, tn);
   float4_t acc[FM][FN];
@@ -1538,12 +1317,12 @@ hipError_t launch_small_code(int code, const GemmParams &p, long batch, hipStrea
   }
 }
 
-template <int BM, int BN, int BK, int WM, int WN, bool TA, bool TB, bool VEC>
+template <int BM, int BN, int BK, int WM, int WN, bool TA, bool TB, bool VEC, bool GATED = false>
 hipError_t launch_f32(GemmParams p, long batch, hipStream_t s) {
   p.tiles_m = (int)((p.M + BM - 1) / BM);
   p.tiles_n = (int)((p.N + BN - 1) / BN);
   dim3 grid((unsigned)(p.tiles_m * p.tiles_n), 1, (unsigned)batch);
-  hipLaunchKernelGGL((gemm_f32_kernel<BM, BN, BK, WM, WN, TA, TB, VEC>), grid, dim3(WM * WN * 64), 0, s, p);
+  hipLaunchKernelGGL((gemm_f32_kernel<BM, BN, BK, WM, WN, TA, TB, VEC, GATED>), grid, dim3(WM * WN * 64), 0, s, p);
   return hipGetLastError();
 }
 
@@ -1556,12 +1335,12 @@ hipError_t launch_f16_ring(GemmParams p, long batch, hipStream_t s) {
   return hipGetLastError();
 }
 
-template <int BM, int BN, int WM, int WN, bool TA, bool TB, int WPE = 2, int NS = 2>
+template <int BM, int BN, int WM, int WN, bool TA, bool TB, int WPE = 2, int NS = 2, bool GATED = false>
 hipError_t launch_f32_ring(GemmParams p, long batch, hipStream_t s) {
   p.tiles_m = (int)((p.M + BM - 1) / BM);
   p.tiles_n = (int)((p.N + BN - 1) / BN);
   dim3 grid((unsigned)(p.tiles_m * p.tiles_n), 1, (unsigned)batch);
-  hipLaunchKernelGGL((gemm_f32_ring_kernel<BM, BN, WM, WN, TA, TB, WPE, NS>), grid, dim3(WM * WN * 64), 0, s, p);
+  hipLaunchKernelGGL((gemm_f32_ring_kernel<BM, BN, WM, WN, TA, TB, WPE, NS, GATED>), grid, dim3(WM * WN * 64), 0, s, p);
   return hipGetLastError();
 }
 
@@ -2032,7 +1811,9 @@ __global__ void gemm_k0_kernel(GemmParams p, long batch) {
 template <bool VST, int ACT>
 __global__ void __launch_bounds__(256)
     splitk_reduce_kernel(const float *__restrict__ P, int S, long PS, long M, long N, float *C, long ldc,
-                         float alpha, float beta, const float *__restrict__ bias, int act_rt, float act_alpha) {
+                         float alpha, float beta, const float *__restrict__ bias, int act_rt, float act_alpha,
+                         const unsigned long long *gate, unsigned long long gate_seq) {
+  if (gate && *gate == gate_seq) return;  // the partials were not written (GemmParams)
   const long MN = M * N;
   const int act = ACT == kActRuntime ? act_rt : ACT;
   const long step = (long)gridDim.x * blockDim.x;
@@ -2080,9 +1861,6 @@ __global__ void __launch_bounds__(256)
   }
 }
 
-// The partials' stride: M x N rounded up to a multiple of 4 floats.
-inline long splitk_stride(long M, long N) { return (M * N + 3) / 4 * 4; }
-
 hipError_t launch_splitk_reduce(const float *P, int S, const GemmParams &p, hipStream_t s) {
   const bool vst = p.N % 4 == 0 && p.ldc % 4 == 0 && ((uintptr_t)p.C & 15) == 0;
   const long groups = (p.M * p.N + 3) / 4;
@@ -2090,7 +1868,7 @@ hipError_t launch_splitk_reduce(const float *P, int S, const GemmParams &p, hipS
   const long PS = splitk_stride(p.M, p.N);
   auto go = [&](auto v, auto a) {
     hipLaunchKernelGGL((splitk_reduce_kernel<decltype(v)::value, decltype(a)::value>), grid, block, 0, s, P, S, PS,
-                       p.M, p.N, p.C, p.ldc, p.alpha, p.beta, p.bias, p.act, p.act_alpha);
+                       p.M, p.N, p.C, p.ldc, p.alpha, p.beta, p.bias, p.act, p.act_alpha, p.gate, p.gate_seq);
   };
   auto pick = [&](auto v) {
     switch (p.act) {
@@ -2120,11 +1898,10 @@ hipError_t launch_splitk_reduce(const float *P, int S, const GemmParams &p, hipS
 // (one round of the two-per-CU tiles), the range its model was checked on: there the split
 // won or tied on every shape measured (2048 x 2048 x 16384: 167 -> 129 us; 2048 x 2048 x 8192:
 // 90 -> 81 us); fp32 takes the model's word.
-int choose_split(int dtype, long M, long N, long K, bool beta) {
-  if (K < 1024 || K % 64) return 1;
+// *us, if asked for, receives the price of the chosen S.
+int choose_split(int dtype, long M, long N, long K, bool beta, double *us = nullptr) {
   const bool f16 = dtype == GN_F16;
   const long tiles128 = ((M + 127) / 128) * ((N + 127) / 128);
-  if (f16 && tiles128 >= 512) return 1;
   auto gemm_us = [&](long S) {
     const double ks = (double)(K / S) / 1024.0;
     if (f16) return f16_best<false>(M, N, S).cost * (ks * 24.9 + 13.8);
@@ -2136,6 +1913,8 @@ int choose_split(int dtype, long M, long N, long K, bool beta) {
   };
   auto reduce_us = [&](long S) { return 2.5 + (double)(S + 1 + (beta ? 1 : 0)) * (double)(M * N) * 4.0 / 5.0e6; };
   const double whole = gemm_us(1);
+  if (us) *us = whole;
+  if (K < 1024 || K % 64 || (f16 && tiles128 >= 512)) return 1;
   double best = whole * (f16 ? 0.9 : 0.95);
   int pick = 1;
   for (long S = 2; S <= 32; ++S) {
@@ -2143,7 +1922,144 @@ int choose_split(int dtype, long M, long N, long K, bool beta) {
     const double t = gemm_us(S) + reduce_us(S);
     if (t < best) best = t, pick = (int)S;
   }
+  if (us && pick > 1) *us = best;
   return pick;
+}
+
+// ------------------------------------------------------------------ fp32 on the bf16 cores
+// csrc/gemm_split.hip computes an fp32 product on the bf16 matrix cores at 1.6 times the speed of
+// the fp32 ones and with a smaller error. The dispatch prices both.
+//
+// The price (us) of an fp32 product on the fp32 matrix cores: the tile model of choose_split, the
+// store of C, the packing of unaligned operands, and the second launch over K % 32.
+double f32_cores_us(const GemmDesc &d, bool a_ok, bool b_ok) {
+  const long Kp = (!a_ok && !b_ok) ? (d.K + 63) / 64 * 64 : d.K;
+  const double c_bytes = 4.0 * (double)d.M * d.N * d.batch;
+  double us = 0;
+  if (d.batch == 1) {
+    choose_split(GN_F32, d.M, d.N, Kp, d.beta != 0.0f, &us);
+  } else {
+    const long tiles64 = ((d.M + 63) / 64) * ((d.N + 63) / 64) * d.batch;
+    us = 219.6 * f32_ring_costs(d.M, d.N, d.batch).best() / 65536.0 * (Kp / 1024.0) * (tiles64 <= 256 ? 1.1 : 1.0);
+  }
+  us += 3.0 + 0.8 * c_bytes / 5.0e6;
+  const double packed = ((a_ok ? 0.0 : (double)d.M) + (b_ok ? 0.0 : (double)d.N)) * (double)d.K * d.batch;
+  if (packed > 0) us += 3.0 + packed * 8.0 / 4.0e6;
+  if (Kp % 32) us += 4.0 + 2.0 * c_bytes / 4.0e6;
+  return us;
+}
+
+// The fp32 kernels behind a split product (GemmParams::gate): 128 x 128 ring tiles and the last
+// K % 32 on the register-staged kernel, or that kernel alone where the ring does not go.
+template <bool TA, bool TB, bool VEC>
+hipError_t launch_f32_behind(const GemmParams &p, long batch, hipStream_t s) {
+  if constexpr (VEC) {
+    if (ring_offsets_fit(p) && p.K >= 32) {
+      const long kt = p.K % 32;
+      GemmParams head = p, tail = p;
+      head.K = p.K - kt;
+      if (kt) {
+        head.bias = nullptr;
+        head.act = -1;
+      }
+      if (hipError_t e = launch_f32_ring<128, 128, 2, 2, TA, TB, 2, 2, true>(head, batch, s)) return e;
+      if (!kt) return hipSuccess;
+      tail.K = kt;
+      tail.beta = 1.0f;
+      tail.A = static_cast<const float *>(p.A) + (TA ? head.K * p.lda : head.K);
+      tail.B = static_cast<const float *>(p.B) + (TB ? head.K : head.K * p.ldb);
+      return launch_f32<64, 64, 16, 2, 2, TA, TB, true, true>(tail, batch, s);
+    }
+  }
+  return launch_f32<64, 64, 16, 2, 2, TA, TB, VEC, true>(p, batch, s);
+}
+
+template <bool VEC>
+hipError_t dispatch_behind(bool ta, bool tb, const GemmParams &p, long batch, hipStream_t s) {
+  if (ta) return tb ? launch_f32_behind<true, true, VEC>(p, batch, s) : launch_f32_behind<true, false, VEC>(p, batch, s);
+  return tb ? launch_f32_behind<false, true, VEC>(p, batch, s) : launch_f32_behind<false, false, VEC>(p, batch, s);
+}
+
+// How a product runs through launch_split within the scratch a stream keeps: nb batches and kc
+// of K at a time (a multiple of 32; later parts of K add to C), each by `plan`.
+struct SplitCut {
+  long nb = 0, kc = 0;
+  SplitPlan plan;
+  size_t ws_bytes = 0;
+};
+
+// true when the product runs on the bf16 matrix cores: priced (the operands' packing, the
+// product, the reduce, 3 us for the fp32 kernels that stand behind it) at least 7% below the
+// fp32 matrix cores. Both prices were checked on 44 shapes (device times, fp32 -> bf16 parts, us):
+// taken 2048 x 2048 x 512 35 -> 35, 4096 x 4096 x 256 73 -> 60, 777 x 1234 x 4099 106 -> 74, 512 x
+// 11008 x 4096 369 -> 332, 2560^3 271 -> 167, 4096^3 928 -> 606; left on the fp32 cores, where the
+// packing or the fixed 15 us weigh too much: 1024^3 21 -> 35, 1280^3 42 -> 42, 256 x 4096 x 4096 71
+// -> 82, 128 x 8192 x 8192 139 -> 255. None of the 44 got slower; of those left, 512 x 4096 x 4096
+// would have gained most (125 -> 114).
+bool cut_split(const GemmDesc &d, bool a_ok, bool b_ok, SplitCut *cut) {
+  constexpr size_t kLimit = kScratchRetainBytes - 512;
+  const bool beta = d.beta != 0.0f;
+  cut->nb = d.batch;
+  cut->kc = d.K;
+  if (!plan_split(d.M, d.N, d.K, d.batch, beta, &cut->plan)) return false;
+  double us = cut->plan.us;
+  size_t bytes = cut->plan.pack_bytes + cut->plan.part_bytes;
+  if (bytes > kLimit && d.batch > 1) {
+    cut->nb = std::max(1L, (long)((double)kLimit / (double)bytes * (double)d.batch));
+    if (!plan_split(d.M, d.N, d.K, cut->nb, beta, &cut->plan)) return false;
+    us = cut->plan.us * (double)d.batch / (double)cut->nb;
+    bytes = cut->plan.pack_bytes + cut->plan.part_bytes;
+  }
+  if (bytes > kLimit) {
+    if (d.batch > 1) return false;
+    const long parts = (long)(bytes / kLimit) + 1;
+    cut->kc = ((d.K + parts - 1) / parts + 31) / 32 * 32;
+    if (cut->kc < 1024 || !plan_split(d.M, d.N, cut->kc, 1, true, &cut->plan)) return false;
+    us = (double)parts * cut->plan.us + (double)(parts - 1) * 8.0 * (double)d.M * d.N / 5.0e6;
+    bytes = cut->plan.pack_bytes + cut->plan.part_bytes;
+    if (bytes > kLimit) return false;
+  }
+  cut->ws_bytes = bytes + 512;  // the gate's block and the partials' rounding up
+  return us + 3.0 < 0.93 * f32_cores_us(d, a_ok, b_ok);
+}
+
+// Enqueues the product by `cut` with ws (cut.ws_bytes) as its workspace. Behind every part the
+// fp32 kernels are enqueued too; they return at once unless an operand holds a value the split
+// does not (an infinity, a NaN, or 2^36 and more), in which case the part's split kernels wrote
+// nothing.
+hipError_t run_split(const GemmDesc &d, const SplitCut &cut, bool vec, char *ws, hipStream_t s) {
+  static std::atomic<unsigned long long> calls{0};
+  auto *gate = reinterpret_cast<unsigned long long *>(ws);
+  float *part = reinterpret_cast<float *>(ws + 256);
+  char *packed = ws + 256 + (cut.plan.part_bytes + 255) / 256 * 256;
+  for (long z = 0; z < d.batch; z += cut.nb)
+    for (long k = 0; k < d.K; k += cut.kc) {
+      GemmDesc q = d;
+      q.batch = std::min(cut.nb, d.batch - z);
+      q.K = std::min(cut.kc, d.K - k);
+      q.A = static_cast<const float *>(d.A) + z * d.strideA + (d.ta ? k * d.lda : k);
+      q.B = static_cast<const float *>(d.B) + z * d.strideB + (d.tb ? k : k * d.ldb);
+      q.C = d.C + z * d.strideC;
+      if (k > 0) q.beta = 1.0f;
+      if (k + cut.kc < d.K) q.bias = nullptr, q.act = -1;
+      SplitPlan plan = cut.plan;
+      plan.S = (int)std::min<long>(plan.S, (q.K + 31) / 32);
+      // a value no earlier call left in *gate; a chance match in fresh scratch only costs time
+      const unsigned long long seq = ++calls;
+      if (hipError_t e = launch_split(q, plan, packed, part, gate, seq, s)) return e;
+      GemmParams p{};
+      p.A = q.A; p.B = q.B; p.C = q.C; p.bias = q.bias;
+      p.M = q.M; p.N = q.N; p.K = q.K;
+      p.lda = q.lda; p.ldb = q.ldb; p.ldc = q.ldc;
+      p.strideA = q.strideA; p.strideB = q.strideB; p.strideC = q.strideC;
+      p.alpha = q.alpha; p.beta = q.beta; p.act = q.act; p.act_alpha = q.act_alpha;
+      p.gate = gate;
+      p.gate_seq = seq;
+      if (plan.S > 1)
+        if (hipError_t e = launch_splitk_reduce(part, plan.S, p, s)) return e;
+      if (hipError_t e = vec ? dispatch_behind<true>(q.ta, q.tb, p, q.batch, s) : dispatch_behind<false>(q.ta, q.tb, p, q.batch, s)) return e;
+    }
+  return hipSuccess;
 }
 
 }  // namespace
@@ -2211,6 +2127,21 @@ int launch_gemm(const GemmDesc &d, hipStream_t s, CError *err) {
     const bool small = gemv || (d.dtype == GN_F32 ? f32_small_tile(d.M, d.N, d.K, d.batch, d.ta, d.tb)
                                           : f16_small_tile(d.M, d.N, d.K, d.batch, d.ta, d.tb)) != 0;
     bool pack = !vec && big && !small && pack_bytes <= ((size_t)4 << 30) && pack_grid_y <= 65535;
+    // A large fp32 product on the bf16 matrix cores (cut_split). Its scratch is not allocated
+    // under graph capture; where the allocation fails the fp32 matrix cores take the product.
+    SplitCut cut;
+    if (d.dtype == GN_F32 && !small && (double)d.M * d.N * d.K * d.batch >= (double)(1L << 29) &&
+        cut_split(d, a_ok, b_ok, &cut)) {
+      hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+      if (hipStreamIsCapturing(s, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone) {
+        std::unique_lock<std::mutex> lk;
+        if (char *ws = static_cast<char *>(stream_scratch(s, cut.ws_bytes, lk, nullptr))) {
+          e = run_split(d, cut, vec, ws, s);
+          stream_scratch_trim(s, lk);
+          return e == hipSuccess ? 0 : hip_error(err, -6, "gemm launch", e);
+        }
+      }
+    }
     // Split-K (choose_split) for a batch-1 product on the aligned path, packed or not, whose
     // operands suit the DMA ring; the partial products take S x M x N floats of the scratch
     // (each M x N rounded up to a multiple of 4), ahead of the packed copies.

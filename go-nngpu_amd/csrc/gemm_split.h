@@ -1,0 +1,35 @@
+// gemm_split.h — large fp32 products on the bf16 matrix cores (gemm_split.hip), called by the
+// GEMM dispatch (gemm.hip).
+#pragma once
+
+#include "common.h"
+
+namespace gn {
+
+// The values the split layout holds: |x| < kSplitMax; the packed parts are of x * kSplitScale.
+constexpr float kSplitScale = 65536.0f;      // 2^16
+constexpr float kSplitMax = 68719476736.0f;  // 2^36
+constexpr int kSplitBlock = 3072;            // bytes of 16 rows x 32 k in three bf16 parts
+constexpr long kSplitMaxK = 1L << 20;        // K up to which no partial sum overflows
+
+// How a product of `batch` M x N x K problems is cut: tile (index into the kernel's shapes), S
+// slices of K, the device time it is priced at (us, pack and reduce included), and the bytes
+// of the packed operands and the partial products.
+struct SplitPlan {
+  int tile = 0, S = 1;
+  double us = 0;
+  size_t pack_bytes = 0, part_bytes = 0;
+};
+// false: a shape the split kernels do not take.
+bool plan_split(long M, long N, long K, long batch, bool beta, SplitPlan *out);
+// The partials' stride in floats: M x N rounded up to a multiple of 4.
+inline long splitk_stride(long M, long N) { return (M * N + 3) / 4 * 4; }
+
+// Packs both operands into ws (plan.pack_bytes) and multiplies them into C (d.C with the
+// epilogue when plan.S == 1, else the partial products of the S slices into part). *gate
+// becomes seq when an operand holds a value the layout does not: the product kernel then
+// writes nothing.
+hipError_t launch_split(const GemmDesc &d, const SplitPlan &plan, char *ws, float *part, unsigned long long *gate,
+                        unsigned long long seq, hipStream_t s);
+
+}  // namespace gn
