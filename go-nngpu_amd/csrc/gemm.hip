@@ -25,6 +25,7 @@
 //  * a grouped, XCD-aware tile order: hardware dispatches workgroup w to XCD w % 8,
 //    so w is remapped to give each XCD a contiguous band of tiles that share A/B
 //    panels in that XCD's L2.
+#include "gemm_rows.h"
 #include "gemm_split.h"
 #include "gemm_tile.h"
 
@@ -1219,90 +1220,6 @@ hipError_t launch_small(GemmParams p, long batch, hipStream_t s) {
   return hipGetLastError();
 }
 
-// ------------------------------------------------------------------ NN products of 1-4 rows (GEMV)
-// C = act(alpha X W + beta C + bias) for X of R <= 4 rows (row-major), W stored K x N
-// (N-contiguous), batch 1: HBM-bound on reading W once, at 2 R flops per W element, so the MFMA
-// layout's 16-row fragments would be mostly padding and the tiled kernels' few column tiles
-// stream W from few CUs. Lane l of a workgroup owns columns n0 + E l .. + E - 1 (4 bytes of each
-// row of W, so a wave's load is 256 contiguous bytes); the KW waves split K into contiguous
-// ranges, each summed in k order with fmaf on the VALU, and the partials are added in LDS in wave
-// order before the epilogue. X's entries are uniform across the workgroup.
-template <typename T, int R, int E, int KW>
-__global__ void __launch_bounds__(KW * 64) gemv_nn_kernel(GemmParams p) {
-  __shared__ float red[KW][R][64 * E];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const long nb = (long)blockIdx.x * 64 * E, n0 = nb + (long)lane * E;
-  const T *__restrict__ W = static_cast<const T *>(p.B);
-  const T *__restrict__ X = static_cast<const T *>(p.A);
-  const long kb = p.K * wave / KW, ke = p.K * (wave + 1) / KW;
-  float acc[R][E];
-#pragma unroll
-  for (int m = 0; m < R; ++m)
-#pragma unroll
-    for (int e = 0; e < E; ++e) acc[m][e] = 0.0f;
-  if (n0 < p.N) {  // N is a multiple of E: the E columns are all inside or all past N
-    typedef T VE __attribute__((ext_vector_type(E == 1 ? 2 : E)));
-    auto step = [&](long k) {
-      T w[E];
-      if constexpr (E == 1) {
-        w[0] = W[k * p.ldb + n0];
-      } else {  // n0 and the pitch are even: one 4-byte load
-        const VE v = *reinterpret_cast<const VE *>(W + k * p.ldb + n0);
-#pragma unroll
-        for (int e = 0; e < E; ++e) w[e] = v[e];
-      }
-#pragma unroll
-      for (int m = 0; m < R; ++m) {
-        const float x = (float)X[m * p.lda + k];
-#pragma unroll
-        for (int e = 0; e < E; ++e) acc[m][e] = fmaf(x, (float)w[e], acc[m][e]);
-      }
-    };
-    long k = kb;
-    for (; k + 8 <= ke; k += 8) {
-#pragma unroll
-      for (int u = 0; u < 8; ++u) step(k + u);
-    }
-    for (; k < ke; ++k) step(k);
-  }
-#pragma unroll
-  for (int m = 0; m < R; ++m)
-#pragma unroll
-    for (int e = 0; e < E; ++e) red[wave][m][lane * E + e] = acc[m][e];
-  __syncthreads();
-  float *C = p.C;
-  for (int o = threadIdx.x; o < R * 64 * E; o += KW * 64) {
-    const int m = o / (64 * E), c = o % (64 * E);
-    const long n = nb + c;
-    if (n >= p.N) continue;
-    float v = red[0][m][c];
-#pragma unroll
-    for (int w = 1; w < KW; ++w) v += red[w][m][c];
-    float *dst = C + m * p.ldc + n;
-    const float old = p.beta != 0.0f ? *dst : 0.0f;
-    *dst = apply_act(p.act, p.alpha * v + p.beta * old + (p.bias ? p.bias[n] : 0.0f), p.act_alpha);
-  }
-}
-
-template <typename T, int R>
-hipError_t launch_gemv_r(const GemmParams &p, hipStream_t s) {
-  constexpr int E = sizeof(T) == 2 ? 2 : 1;  // 4 bytes per lane and row of W
-  const unsigned grid = (unsigned)((p.N + 64 * E - 1) / (64 * E));
-  hipLaunchKernelGGL((gemv_nn_kernel<T, R, E, 16>), dim3(grid), dim3(1024), 0, s, p);
-  return hipGetLastError();
-}
-
-// The NN GEMV kernel for a product of M <= 4 rows (batch 1, W aligned, N a multiple of 4 or 8).
-template <typename T>
-hipError_t launch_gemv(const GemmParams &p, hipStream_t s) {
-  switch (p.M) {
-    case 1: return launch_gemv_r<T, 1>(p, s);
-    case 2: return launch_gemv_r<T, 2>(p, s);
-    case 3: return launch_gemv_r<T, 3>(p, s);
-    default: return launch_gemv_r<T, 4>(p, s);
-  }
-}
-
 // The small-product kernel of shape code 100 KW + 10 FM + FN; hipErrorInvalidValue for
 // another code.
 template <typename T, bool TA, bool TB, bool VEC>
@@ -1442,36 +1359,9 @@ hipError_t launch_f16_tile(const GemmParams &p, long batch, hipStream_t s, F16Ti
   }
 }
 
-// NN products of at most 4 rows (batch 1) take the GEMV kernel where it measured faster than the
-// tiled and small-product kernels on a grid of M 1-4, N 512-32768, K 512-11008 (kernel times,
-// tiled -> GEMV): fp32 1 x 11008 x 4096 54.4 -> 28.5 us (6.3 TB/s of W), 2 x 16384 x 2048 37.3 ->
-// 21.0 us, 4 x 11008 x 4096 54.9 -> 43.4 us, 1 x 4096 x 4096 24.8 -> 20.2 us; fp16 1 x 16384 x
-// 2048 18.2 -> 12.1 us, 2 x 2048 x 2048 16.8 -> 9.7 us, 4 x 32768 x 1024 15.2 -> 12.1 us. With
-// fewer columns its grid has too few workgroups (N / 64 or N / 128 of them) and with more rows
-// the VALU work grows: fp32 2 x 4096 x 11008 52.8 against 70.0 us, fp16 4 x 4096 x 4096 13.7
-// against 27.1 us stay on the other kernels.
-inline bool gemv_nn(long M, long N, long K, long batch, bool f16) {
-  if (batch != 1 || M > 4) return false;
-  if (!f16) return N >= 11008 || (M <= 2 && N >= 8192) || (M == 1 && N >= 4096);
-  if (M <= 2 && (N >= 8192 || (N >= 1024 && N <= 2048 && K >= 1024))) return true;
-  return N >= 16384;
-}
-
-// Skinny products in the linear-layer layout Y = X W^T (A row-major, B = W stored N x K,
-// K-contiguous; at most 16 rows, batch 1, N and K of 2048 and more) are bound by reading W
-// once from HBM. The small-product kernel with 16 x 16 tiles reads each W element once, as one
-// 16-byte vector per lane and K step, and each tile's A rows from L2, and its K-splitting waves
-// keep more loads in flight than the tiled kernels' few workgroups: up to 4096 waves (16 per
-// workgroup while ceil(N / 16) <= 256, 8 while <= 512, else 4). Kernel times on MI355X (tiled
-// -> this): fp32 1 x 11008 x 4096 54.9 -> 33.9 us (5.3 TB/s of W), 8 x 4096 x 8192 38.9 ->
-// 28.4 us, 16 x 16384 x 4096 81.8 -> 63.5 us; fp16 1 x 4096 x 2048 17.0 -> 6.1 us, 2 x 11008 x
-// 4096 22.1 -> 16.5 us, 16 x 4096 x 4096 14.0 -> 10.4 us. The bounds leave out the shapes where
-// it lost on a grid of M 1-16, N 2048-16384, K 2048-8192: fp32 past 2 rows needs N >= 4096 (16 x
-// 2048 x 8192: 25.6 against 31.6 us) and M N K < 2^31; fp16 past 2 rows needs M N <= 65536 and
-// K <= 4096 (8 x 16384 x 8192: 45.8 against 50.5 us). With W stored K x N (NN) the kernel's W
-// loads are 4- or 2-byte scalars and it ran 1.1-5x slower than the tiled kernels, so other
-// layouts keep them; a skinny NT product therefore differs from the same product in NN in its
-// rounding (K summed in four to sixteen wave ranges), both within the fp32 bar.
+// Products of at most 16 rows in the linear-layer layout Y = X W^T whose alignment gemm_rows.hip
+// does not take (N and K of 2048 and more, batch 1): the small-product kernel with 16 x 16 tiles
+// and up to 4096 waves reads each W element once, where packing W would write and read it again.
 inline int skinny_tile(long M, long N, long K, long batch, bool f16, bool ta, bool tb) {
   if (ta || !tb || batch != 1 || M > 16 || N < 2048 || K < 2048) return 0;
   if (M > 2) {
@@ -1980,6 +1870,21 @@ hipError_t dispatch_behind(bool ta, bool tb, const GemmParams &p, long batch, hi
   return tb ? launch_f32_behind<false, true, VEC>(p, batch, s) : launch_f32_behind<false, false, VEC>(p, batch, s);
 }
 
+// Where gemm_rows.hip takes a product it can (plan_rows): always up to 16 rows; up to 32 from 2^20
+// elements of W, in fp16 below 2^25 (28 rows x 11008 x 4096: 28.9 us against 27.7 on the split-K
+// ring); up to 64 in fp16 from 2^20 to 12 M elements (64 x 4096 x 1024: 12.7 -> 7.9 us; at 16 M
+// level, at 45 M 36 against 30), in fp32 by price (the fp32 tiles' is for a
+// warm W and 15% low with W from HBM: 40 x 11008 x 4096 74 -> 59), and instead of the small-product
+// kernel for K of 2048 and more (64 x 256 x 4096: 17.2 -> 11.3 us; 64 x 512 x 512: 8.1 against 5.0).
+bool takes_rows(const GemmDesc &d, const RowsPlan &rows, bool a_ok, bool b_ok, bool small) {
+  if (d.M <= 16) return true;
+  const double w = (double)d.N * (double)d.K;
+  if (w < (double)(1L << 20)) return false;
+  if (d.dtype == GN_F16) return w < (d.M <= 32 ? (double)(1L << 25) : 12.0e6);
+  if (d.M <= 32) return true;
+  return small ? d.K >= 2048 : rows.us < 1.15 * (f32_cores_us(d, a_ok, b_ok) + 3.0);
+}
+
 // How a product runs through launch_split within the scratch a stream keeps: nb batches and kc
 // of K at a time (a multiple of 32; later parts of K add to C), each by `plan`.
 struct SplitCut {
@@ -2117,16 +2022,30 @@ int launch_gemm(const GemmDesc &d, hipStream_t s, CError *err) {
     const long Kp = (d.K + 63) / 64 * 64;
     const bool a_ok = aligned(d.A, d.lda, d.strideA) && a_contig % epv == 0;
     const bool b_ok = aligned(d.B, d.ldb, d.strideB) && b_contig % epv == 0;
-    // NN products of 1-4 rows on the GEMV kernel, which needs only W aligned (X is read element
-    // by element)
-    const bool gemv = b_ok && !d.ta && !d.tb && gemv_nn(d.M, d.N, d.K, d.batch, d.dtype == GN_F16);
     const size_t pack_bytes =
         (size_t)((a_ok ? 0 : d.M) + (b_ok ? 0 : d.N)) * (size_t)Kp * esz * (size_t)std::min(kMaxZ, d.batch);
     const bool big = (double)d.M * d.N * d.K >= (double)(1L << 24);
     const long pack_grid_y = (a_ok ? 0 : (d.M + 63) / 64) + (b_ok ? 0 : (d.N + 63) / 64);
-    const bool small = gemv || (d.dtype == GN_F32 ? f32_small_tile(d.M, d.N, d.K, d.batch, d.ta, d.tb)
+    const bool small = (d.dtype == GN_F32 ? f32_small_tile(d.M, d.N, d.K, d.batch, d.ta, d.tb)
                                           : f16_small_tile(d.M, d.N, d.K, d.batch, d.ta, d.tb)) != 0;
     bool pack = !vec && big && !small && pack_bytes <= ((size_t)4 << 30) && pack_grid_y <= 65535;
+    // A product of at most 64 rows (takes_rows), slices of K only outside graph capture (their
+    // partial products take scratch) and where the scratch can be had.
+    RowsPlan rows;
+    if (d.M <= 64 && d.batch == 1 && plan_rows(d, true, &rows) && takes_rows(d, rows, a_ok, b_ok, small)) {
+      std::unique_lock<std::mutex> lk;
+      float *part = nullptr;
+      if (rows.S > 1) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(s, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone)
+          part = static_cast<float *>(stream_scratch(s, rows.part_bytes, lk, nullptr));
+        if (!part) plan_rows(d, false, &rows);
+      }
+      e = launch_rows(d, rows, part, s);
+      if (e == hipSuccess && rows.S > 1) e = launch_splitk_reduce(part, rows.S, p, s);
+      if (lk.owns_lock()) stream_scratch_trim(s, lk);
+      return e == hipSuccess ? 0 : hip_error(err, -6, "gemm launch", e);
+    }
     // A large fp32 product on the bf16 matrix cores (cut_split). Its scratch is not allocated
     // under graph capture; where the allocation fails the fp32 matrix cores take the product.
     SplitCut cut;
@@ -2169,10 +2088,6 @@ int launch_gemm(const GemmDesc &d, hipStream_t s, CError *err) {
       q.B = static_cast<const char *>(d.B) + z0 * d.strideB * (long)esz;
       q.C = d.C + z0 * d.strideC;
       const long nb = std::min(kMaxZ, d.batch - z0);
-      if (gemv) {
-        e = d.dtype == GN_F16 ? launch_gemv<_Float16>(q, s) : launch_gemv<float>(q, s);
-        continue;
-      }
       if (!pack && S == 1) {
         e = vec ? dispatch<true>(d, q, nb, s) : dispatch<false>(d, q, nb, s);
         continue;

@@ -1,0 +1,21 @@
+// gemm_rows.h — products of at most 64 rows (gemm_rows.hip), called by the GEMM dispatch (gemm.hip).
+#pragma once
+
+#include "common.h"
+#include "gemm_split.h"  // splitk_stride
+
+namespace gn {
+
+// Columns per workgroup (16 fn), slices of K across workgroups, the price in us, and the bytes of
+// the slices' partial products.
+struct RowsPlan {
+  int fn = 0, S = 1;
+  double us = 0;
+  size_t part_bytes = 0;
+};
+// false: a shape, layout or alignment these kernels do not take. split_ok: S > 1 is allowed.
+bool plan_rows(const GemmDesc &d, bool split_ok, RowsPlan *out);
+// C with the epilogue (plan.S == 1) or the partial products of the slices into part.
+hipError_t launch_rows(const GemmDesc &d, const RowsPlan &plan, float *part, hipStream_t s);
+
+}  // namespace gn
