@@ -1902,30 +1902,34 @@ struct SplitCut {
 // -> 82, 128 x 8192 x 8192 139 -> 255. None of the 44 got slower; of those left, 512 x 4096 x 4096
 // would have gained most (125 -> 114).
 bool cut_split(const GemmDesc &d, bool a_ok, bool b_ok, SplitCut *cut) {
-  constexpr size_t kLimit = kScratchRetainBytes - 512;
-  const bool beta = d.beta != 0.0f;
-  cut->nb = d.batch;
-  cut->kc = d.K;
-  if (!plan_split(d.M, d.N, d.K, d.batch, beta, &cut->plan)) return false;
+  constexpr size_t kLimit = kScratchRetainBytes - 512;  // less the gate's block and the partials' rounding up
+  GemmDesc q = d;
+  if (!plan_split(q, &cut->plan)) return false;
   double us = cut->plan.us;
   size_t bytes = cut->plan.pack_bytes + cut->plan.part_bytes;
   if (bytes > kLimit && d.batch > 1) {
-    cut->nb = std::max(1L, (long)((double)kLimit / (double)bytes * (double)d.batch));
-    if (!plan_split(d.M, d.N, d.K, cut->nb, beta, &cut->plan)) return false;
-    us = cut->plan.us * (double)d.batch / (double)cut->nb;
+    q.batch = std::max(1L, (long)((double)kLimit / (double)bytes * (double)d.batch));
+    if (!plan_split(q, &cut->plan)) return false;
+    us = cut->plan.us * (double)d.batch / (double)q.batch;
     bytes = cut->plan.pack_bytes + cut->plan.part_bytes;
   }
   if (bytes > kLimit) {
     if (d.batch > 1) return false;
     const long parts = (long)(bytes / kLimit) + 1;
-    cut->kc = ((d.K + parts - 1) / parts + 31) / 32 * 32;
-    if (cut->kc < 1024 || !plan_split(d.M, d.N, cut->kc, 1, true, &cut->plan)) return false;
+    q.K = ((d.K + parts - 1) / parts + 31) / 32 * 32;
+    q.beta = 1.0f;
+    if (q.K < 1024 || !plan_split(q, &cut->plan)) return false;
+    if (cut->plan.raw_b && d.K % 4) return false;  // the last part's K is not the planned one
     us = (double)parts * cut->plan.us + (double)(parts - 1) * 8.0 * (double)d.M * d.N / 5.0e6;
     bytes = cut->plan.pack_bytes + cut->plan.part_bytes;
     if (bytes > kLimit) return false;
   }
-  cut->ws_bytes = bytes + 512;  // the gate's block and the partials' rounding up
-  return us + 3.0 < 0.93 * f32_cores_us(d, a_ok, b_ok);
+  cut->nb = q.batch;
+  cut->kc = q.K;
+  cut->ws_bytes = bytes + 512;
+  // (the fp32 tiles' prices are for operands in the caches: with B from HBM the tiles of a few row
+  // blocks, where a raw B is the choice, took 15-30% more)
+  return us + 3.0 < (cut->plan.raw_b ? 1.0 : 0.93) * f32_cores_us(d, a_ok, b_ok);
 }
 
 // Enqueues the product by `cut` with ws (cut.ws_bytes) as its workspace. Behind every part the
@@ -2049,7 +2053,7 @@ int launch_gemm(const GemmDesc &d, hipStream_t s, CError *err) {
     // A large fp32 product on the bf16 matrix cores (cut_split). Its scratch is not allocated
     // under graph capture; where the allocation fails the fp32 matrix cores take the product.
     SplitCut cut;
-    if (d.dtype == GN_F32 && !small && (double)d.M * d.N * d.K * d.batch >= (double)(1L << 29) &&
+    if (d.dtype == GN_F32 && !small && (double)d.M * d.N * d.K * d.batch >= (double)(1L << 28) &&
         cut_split(d, a_ok, b_ok, &cut)) {
       hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
       if (hipStreamIsCapturing(s, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone) {

@@ -17,18 +17,19 @@ constexpr long kSplitMaxK = 1L << 20;        // K up to which no partial sum ove
 // of the packed operands and the partial products.
 struct SplitPlan {
   int tile = 0, S = 1;
+  bool raw_b = false;  // B is split by the product kernel instead of packed
   double us = 0;
   size_t pack_bytes = 0, part_bytes = 0;
 };
 // false: a shape the split kernels do not take.
-bool plan_split(long M, long N, long K, long batch, bool beta, SplitPlan *out);
+bool plan_split(const GemmDesc &d, SplitPlan *out);
 // The partials' stride in floats: M x N rounded up to a multiple of 4.
 inline long splitk_stride(long M, long N) { return (M * N + 3) / 4 * 4; }
 
-// Packs both operands into ws (plan.pack_bytes) and multiplies them into C (d.C with the
+// Packs the operands into ws (plan.pack_bytes) and multiplies them into C (d.C with the
 // epilogue when plan.S == 1, else the partial products of the S slices into part). *gate
-// becomes seq when an operand holds a value the layout does not: the product kernel then
-// writes nothing.
+// becomes seq when an operand holds a value the parts do not. Then d.C still holds what it held,
+// except with a raw B and S == 1 (which plan_split gives for beta == 0 only).
 hipError_t launch_split(const GemmDesc &d, const SplitPlan &plan, char *ws, float *part, unsigned long long *gate,
                         unsigned long long seq, hipStream_t s);
 

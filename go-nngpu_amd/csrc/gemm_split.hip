@@ -56,20 +56,23 @@ struct Parts {
   bf16x8_t p[3];
 };
 
+// Element e of the three parts of x; bad |= x is none that they hold.
+__device__ __forceinline__ void split1(float x, Parts &o, int e, bool &bad) {
+  bad |= !(fabsf(x) < kSplitMax);
+  const float v = x * kSplitScale;
+  const __bf16 h = (__bf16)v;
+  const float r1 = v - (float)h;
+  const __bf16 m = (__bf16)r1;
+  const float r2 = r1 - (float)m;
+  o.p[0][e] = h;
+  o.p[1][e] = m;
+  o.p[2][e] = (__bf16)r2;
+}
+
 __device__ __forceinline__ Parts split8(const float (&x)[8], bool &bad) {
   Parts o;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    bad |= !(fabsf(x[e]) < kSplitMax);
-    const float v = x[e] * kSplitScale;
-    const __bf16 h = (__bf16)v;
-    const float r1 = v - (float)h;
-    const __bf16 m = (__bf16)r1;
-    const float r2 = r1 - (float)m;
-    o.p[0][e] = h;
-    o.p[1][e] = m;
-    o.p[2][e] = (__bf16)r2;
-  }
+  for (int e = 0; e < 8; ++e) split1(x[e], o, e, bad);
   return o;
 }
 
@@ -129,7 +132,8 @@ __device__ __forceinline__ void dma16s(const BufRsrc &s, unsigned voff, unsigned
       : "memory");
 }
 
-// C tile of BM x BN by WM x WN waves over the K-tiles of a slice. Per 32-k tile a wave multiplies six
+// C tile of BM x BN by WM x WN waves over the K-tiles of a slice; BSRC 0: both operands packed, else
+// B is split here (see "A raw B"). Per 32-k tile a wave multiplies six
 // pairs of part planes (FM x FN MFMAs each); a plane's fragments are read while the two products
 // before its first use run, so at most five of the six planes are in registers beside the two
 // accumulator sets: 239 of 256 registers with 64 x 64 per wave (all six: 254 and spills). The
@@ -141,15 +145,16 @@ __device__ __forceinline__ void dma16s(const BufRsrc &s, unsigned voff, unsigned
 //    workgroup and K-tile); 144 KiB of LDS;
 //  * 128 x 128, 8 waves of 64 x 32: twice the tiles where those leave CUs idle (2048^3: 70 us
 //    against 109); three ring slots measured 1-2% slower than two.
-template <int BM, int BN, int WM, int WN, int NS>
-__global__ void __launch_bounds__(WM * WN * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
+template <int BM, int BN, int WM, int WN, int BSRC, int RD, int WPE>
+__global__ void __launch_bounds__(WM * WN * 64) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
 gemm_split_kernel(GemmParams p, SplitArgs q) {
-  constexpr int NW = WM * WN, FM = BM / WM / 16, FN = BN / WN / 16;
+  constexpr int NW = WM * WN, FM = BM / WM / 16, FN = BN / WN / 16, NS = 2;
   constexpr int CA = BM / 16 * 3, CB = BN / 16 * 3;  // 1 KiB chunks of a K-tile of A and of B
-  constexpr int IPA = CA / NW, IPB = CB / NW, LPW = IPA + IPB;
+  constexpr int IPA = (CA + NW - 1) / NW, IPB = BSRC ? 0 : CB / NW, LPW = IPA + IPB;
+  static_assert(RD == 1 || RD == 2, "raw buffers");
+  static_assert(BSRC == 0 || (BN == 128 && NW == 8), "a raw B: one 16-column block, or 64 columns x 8 k, per wave");
   constexpr int SLOT = (CA + CB) * 1024;
-  static_assert(CA % NW == 0 && CB % NW == 0, "tile shape");
-  static_assert(NS == 2, "the wait before the barrier is for every copy in flight");
+  static_assert((CA % NW == 0 || CA < 2 * NW) && CB % NW == 0, "tile shape");
   static_assert(WM * 16 * (BN + 4) * 4 <= NS * SLOT, "epilogue staging exceeds the ring");
   __shared__ __attribute__((aligned(1024))) char smem[NS * SLOT];
   if (*p.gate == p.gate_seq) return;  // uniform: a value the split does not hold; the fp32 kernels run instead
@@ -165,10 +170,11 @@ gemm_split_kernel(GemmParams p, SplitArgs q) {
   const BufRsrc rb = make_rsrc(static_cast<const char *>(p.B) + zb * q.sb);
   const unsigned sbase = lds_offset(smem);
   const unsigned voff = lane * 16;
-  unsigned soa[IPA], sob[IPB];
+  unsigned soa[IPA], sob[IPB ? IPB : 1];
 #pragma unroll
   for (int i = 0; i < IPA; ++i) {
-    const int c = wave * IPA + i, blk = min((int)(m0 >> 4) + c / 3, q.nra - 1);
+    // (with 12 chunks for 8 waves the last ones copy chunk 11 again)
+    const int c = min(wave * IPA + i, CA - 1), blk = min((int)(m0 >> 4) + c / 3, q.nra - 1);
     soa[i] = (unsigned)blk * (unsigned)q.nkt * kSplitBlock + (unsigned)kt0 * kSplitBlock + (c % 3) * 1024;
   }
 #pragma unroll
@@ -183,12 +189,46 @@ gemm_split_kernel(GemmParams p, SplitArgs q) {
     for (int i = 0; i < IPA; ++i)
       if (2 * i / LPW == h)
         dma16s(ra, voff, __builtin_amdgcn_readfirstlane(soa[i] + ko),
-               __builtin_amdgcn_readfirstlane(st + (wave * IPA + i) * 1024));
+               __builtin_amdgcn_readfirstlane(st + min(wave * IPA + i, CA - 1) * 1024));
 #pragma unroll
     for (int i = 0; i < IPB; ++i)
       if (2 * (IPA + i) / LPW == h)
         dma16s(rb, voff, __builtin_amdgcn_readfirstlane(sob[i] + ko),
                __builtin_amdgcn_readfirstlane(st + (CA + wave * IPB + i) * 1024));
+  };
+  // A raw B (BSRC 1: K-contiguous, rows of whole 16-byte vectors; 2: N-contiguous): a thread loads
+  // eight k of one column of a K-tile into registers, NS + RD K-tiles ahead of their multiplication,
+  // and writes their parts into the slot NS K-tiles ahead of it. Every K-tile takes RAW
+  // unconditional load instructions, which the waits count on: columns past N are the last
+  // one's (multiplied and not stored), k past K is some k before it (A's parts are zero there).
+  constexpr int RAW = BSRC == 1 ? 2 : 8;
+  constexpr bool MIX = FM * FN <= 8;  // the splits run beside MFMAs where the registers allow it
+  const int bg = BSRC == 1 ? lane >> 4 : wave >> 1, bcol = BSRC == 1 ? wave * 16 + (lane & 15) : (wave & 1) * 64 + lane;
+  const float *bsrc = static_cast<const float *>(p.B) + zb * p.strideB;
+  const long blane = min(n0 + bcol, p.N - 1) * (BSRC == 1 ? p.ldb : 1);
+  float raw[RD][8];
+  bool bad = false;
+  auto load_raw = [&](int r, int t) {
+    const long k = (long)(kt0 + t) * 32 + 8 * bg;
+    if (BSRC == 1) {
+      const float4_t u = *reinterpret_cast<const float4_t *>(bsrc + blane + min(k, p.K - 4));
+      const float4_t v = *reinterpret_cast<const float4_t *>(bsrc + blane + min(k + 4, p.K - 4));
+#pragma unroll
+      for (int e = 0; e < 4; ++e) raw[r][e] = u[e], raw[r][4 + e] = v[e];
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) raw[r][e] = bsrc[min(k + e, p.K - 1) * p.ldb + blane];
+    }
+  };
+  Parts parts;
+  auto split_raw = [&](int r, int e0, int e1) {
+#pragma unroll
+    for (int e = e0; e < e1; ++e) split1(raw[r][e], parts, e, bad);
+  };
+  auto write_raw = [&](int slot) {
+    char *d = smem + slot * SLOT + (CA + (bcol >> 4) * 3) * 1024 + (bg * 16 + (bcol & 15)) * 16;
+#pragma unroll
+    for (int h = 0; h < 3; ++h) *reinterpret_cast<bf16x8_t *>(d + h * 1024) = parts.p[h];
   };
   bf16x8_t fa[FM][3], fb[FN][3];
   auto read_a = [&](int slot, int h) {
@@ -220,16 +260,25 @@ gemm_split_kernel(GemmParams p, SplitArgs q) {
     if (u < nt) {
       issue(u, u, 0);
       issue(u, u, 1);
+      if (BSRC) {
+        load_raw(0, u);
+        split_raw(0, 0, 8);
+        write_raw(u);
+      }
     }
-  if (nt >= NS) __builtin_amdgcn_s_waitcnt(vmcnt_imm((NS - 1) * LPW));
+#pragma unroll
+  for (int r = 0; BSRC && r < RD; ++r) load_raw(r, NS + r);
+  if (BSRC) __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+  else if (nt >= NS) __builtin_amdgcn_s_waitcnt(vmcnt_imm((NS - 1) * LPW));
   else __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
   __syncthreads();
   read_b(0, 1);
   read_a(0, 1);
   read_b(0, 2);
   int cur = 0;
-  for (int t = 0; t < nt; ++t) {
-    const int nxt = cur + 1 == NS ? 0 : cur + 1;
+  auto step = [&](int t, int r) {  // r: the raw buffer of K-tile t + NS
+    const int nxt = cur ^ 1;
+    const bool more = t + NS < nt;
     __builtin_amdgcn_sched_barrier(0);
     read_a(cur, 0);
     mul(1, 1);
@@ -243,27 +292,57 @@ gemm_split_kernel(GemmParams p, SplitArgs q) {
     mul(0, 2);
     sched_interleave<FM * FN, FM>();
     __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));  // K-tile t + 1
+    // the copies of K-tile t + 1; a raw B's newest loads, issued behind them, may still be in flight
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(BSRC ? RAW : 0));
     __syncthreads();
+    if (BSRC) {
+      // raw[r] is waited for here: behind the next copies the compiler's wait would be for those too
+#pragma unroll
+      for (int e = 0; e < 8; ++e) asm volatile("" : "+v"(raw[r][e]));
+    }
     __builtin_amdgcn_sched_barrier(0);
-    if (t + NS < nt) issue(t + NS, cur, 0);
+    if (more) issue(t + NS, cur, 0);
     __builtin_amdgcn_sched_barrier(0);
     read_b(nxt, 1);
+    if (BSRC && MIX) split_raw(r, 0, 4);
     mul(2, 0);
-    sched_interleave<FM * FN, FN>();
+    if (BSRC && MIX) sched_mix<FM * FN, FN>();
+    else sched_interleave<FM * FN, FN>();
     __builtin_amdgcn_sched_barrier(0);
-    if (t + NS < nt) issue(t + NS, cur, 1);
+    if (more) issue(t + NS, cur, 1);
+    if (BSRC && !MIX) {
+      split_raw(r, 0, 8);
+      write_raw(cur);
+    }
     __builtin_amdgcn_sched_barrier(0);
     read_b(nxt, 2);
+    if (BSRC && MIX) {
+      split_raw(r, 4, 8);
+      write_raw(cur);
+    }
     mul(1, 0);
-    sched_interleave<FM * FN, FN>();
+    if (BSRC && MIX) sched_mix<FM * FN, FN>();
+    else sched_interleave<FM * FN, FN>();
+    __builtin_amdgcn_sched_barrier(0);
+    if (BSRC) load_raw(r, t + NS + RD);
     __builtin_amdgcn_sched_barrier(0);
     read_a(nxt, 1);
     mul(0, 0);
     sched_interleave<FM * FN, FM>();
     cur = nxt;
+  };
+  if constexpr (BSRC && RD == 2) {
+    int t = 0;
+    for (; t + 1 < nt; t += 2) {
+      step(t, 0);
+      step(t + 1, 1);
+    }
+    if (t < nt) step(t, 0);
+  } else {
+    for (int t = 0; t < nt; ++t) step(t, 0);
   }
   __syncthreads();
+  if (BSRC && bad) *const_cast<unsigned long long *>(p.gate) = p.gate_seq;
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
@@ -271,49 +350,70 @@ gemm_split_kernel(GemmParams p, SplitArgs q) {
   store_tile_rows<BM, BN, WM, WN>(p, m0, n0, z, reinterpret_cast<float *>(smem), acc);
 }
 
-template <int BM, int BN, int WM, int WN, int NS>
+template <int BM, int BN, int WM, int WN, int BSRC = 0, int RD = 1, int WPE = 2>
 hipError_t launch_tile(GemmParams p, const SplitArgs &q, long batch, hipStream_t s) {
   p.tiles_m = (int)((p.M + BM - 1) / BM);
   p.tiles_n = (int)((p.N + BN - 1) / BN);
   const dim3 grid((unsigned)(p.tiles_m * p.tiles_n), 1, (unsigned)(batch * q.S));
-  hipLaunchKernelGGL((gemm_split_kernel<BM, BN, WM, WN, NS>), grid, dim3(WM * WN * 64), 0, s, p, q);
+  hipLaunchKernelGGL((gemm_split_kernel<BM, BN, WM, WN, BSRC, RD, WPE>), grid, dim3(WM * WN * 64), 0, s, p, q);
   return hipGetLastError();
 }
 
-hipError_t launch_shape(int tile, const GemmParams &p, const SplitArgs &q, long batch, hipStream_t s) {
-  return tile == 0 ? launch_tile<256, 128, 4, 2, 2>(p, q, batch, s) : launch_tile<128, 128, 2, 4, 2>(p, q, batch, s);
+hipError_t launch_shape(const SplitPlan &plan, int bsrc, const GemmParams &p, const SplitArgs &q, long batch,
+                        hipStream_t s) {
+  if (bsrc == 1)
+    return plan.tile == 0 ? launch_tile<256, 128, 4, 2, 1, 1>(p, q, batch, s) : launch_tile<128, 128, 2, 4, 1, 2>(p, q, batch, s);
+  if (bsrc == 2)
+    return plan.tile == 0 ? launch_tile<256, 128, 4, 2, 2, 1>(p, q, batch, s) : launch_tile<128, 128, 2, 4, 2, 2>(p, q, batch, s);
+  return plan.tile == 0 ? launch_tile<256, 128, 4, 2>(p, q, batch, s) : launch_tile<128, 128, 2, 4>(p, q, batch, s);
 }
 
 long blocks16(long n) { return (n + 15) / 16; }
 
+bool vectors(const void *ptr, long ld, long stride, long batch) {
+  return (uintptr_t)ptr % 16 == 0 && ld % 4 == 0 && (batch == 1 || stride % 4 == 0);
+}
+
 }  // namespace
 
-bool plan_split(long M, long N, long K, long batch, bool beta, SplitPlan *out) {
-  const long nkt = (K + 31) / 32;
+bool plan_split(const GemmDesc &d, SplitPlan *out) {
+  const long M = d.M, N = d.N, K = d.K, batch = d.batch, nkt = (K + 31) / 32;
+  const bool beta = d.beta != 0.0f;
   if (K < 32 || K > kSplitMaxK || batch > 16384 || (M + 63) / 64 + (N + 63) / 64 > 65535) return false;
   const size_t pa = (size_t)blocks16(M) * nkt * kSplitBlock, pb = (size_t)blocks16(N) * nkt * kSplitBlock;
-  if (pa >= ring::kNumRecords || pb >= ring::kNumRecords) return false;  // 32-bit copy offsets
-  // Prices in us, fitted to 44 shapes (64 x 8192 x 8192 to 8192 x 8192 x 128, both tiles, S 1-16; within
-  // 15%): the pack at 4.6 TB/s, a round of 256 workgroups at a fixed part (launch, first copies, the
-  // store of C) plus its K-tiles, which cost more the more CUs share the board's power, and the
-  // reduce. Slices keep at least 8 K-tiles.
-  const double pack_us = 3.0 + (double)batch * (double)(M + N) * (double)K * 10.0 / 4.6e6;
+  if (pa >= ring::kNumRecords) return false;  // 32-bit copy offsets
+  // Prices in us, fitted to 44 shapes (64 x 8192 x 8192 to 8192 x 8192 x 128, both tiles, S 1-16) and 13
+  // with a raw B, within 15%: the packing at 4.6 TB/s, a round of 256 workgroups at a fixed part (launch,
+  // first copies, the store of C) plus its K-tiles, which cost more the more CUs share the board's
+  // power, and the reduce. Slices keep at least 8 K-tiles. A raw B saves its packing (10 bytes per
+  // element) and costs a 256-row tile's K-tile about a tenth, a 128-row tile's half as much again: it
+  // pays for up to about 512 rows (512 x 11008 x 4096 NT 323 -> 250 us, 256 rows 217 -> 156; 1024 x 4096 x
+  // 1024: level). It reads 16-byte vectors of a K-contiguous B.
+  const bool raw_ok = d.tb ? vectors(d.B, d.ldb, d.strideB, batch) && K % 4 == 0 : true;
   out->us = 1e30;
-  for (int tile = 0; tile < 2; ++tile) {
+  for (int form = 0; form < 4; ++form) {
+    const int tile = form & 1;
+    const bool raw = form >= 2;
+    if (raw ? !raw_ok : pb >= ring::kNumRecords) continue;
+    const double pack_us = 3.0 + (double)batch * (double)(M + (raw ? 0 : N)) * (double)K * 10.0 / 4.6e6;
+    const double w_us = raw ? (double)batch * (double)N * (double)K * 4.0 / 4.9e6 : 0.0;
     const long bm = tile == 0 ? 256 : 128;
     const long tiles = ((M + bm - 1) / bm) * ((N + 127) / 128) * batch;
     if (tiles > (1L << 30)) return false;
     for (long S = 1; S <= (batch == 1 ? 32 : 1) && S <= nkt; ++S) {
       if (S > 1 && nkt / S < 8) break;
+      if (raw && S == 1 && beta) continue;
       const long w = tiles * S, rounds = (w + 255) / 256;
       const double kt = (double)((nkt + S - 1) / S), busy = (double)w / (256.0 * (double)rounds);
-      const double wg = tile == 0 ? 9.0 + (1.54 + 0.36 * busy) * kt : 8.0 + (0.66 + 0.26 * busy) * kt;
-      const double us = pack_us + (double)rounds * wg +
+      const double wg = raw ? (tile == 0 ? 10.0 + (1.75 + 0.6 * busy) * kt : 8.0 + 1.36 * kt)
+                            : tile == 0 ? 9.0 + (1.54 + 0.36 * busy) * kt : 8.0 + (0.66 + 0.26 * busy) * kt;
+      const double us = pack_us + std::max((double)rounds * wg, w_us) +
                         (S > 1 ? 2.5 + (double)(S + 1 + (beta ? 1 : 0)) * (double)(M * N) * 4.0 / 5.0e6 : 0.0);
-      if (us < out->us) out->us = us, out->tile = tile, out->S = (int)S;
+      if (us < out->us) out->us = us, out->tile = tile, out->S = (int)S, out->raw_b = raw;
     }
   }
-  out->pack_bytes = (size_t)batch * (pa + pb);
+  if (out->us >= 1e30) return false;
+  out->pack_bytes = (size_t)batch * (pa + (out->raw_b ? 0 : pb));
   out->part_bytes = out->S > 1 ? (size_t)out->S * splitk_stride(M, N) * sizeof(float) : 0;
   return true;
 }
@@ -328,18 +428,19 @@ hipError_t launch_split(const GemmDesc &d, const SplitPlan &plan, char *ws, floa
   q.sa = (long)q.nra * q.nkt * kSplitBlock;
   q.sb = (long)q.nrb * q.nkt * kSplitBlock;
   char *pb = ws + d.batch * q.sa;
-  auto vec = [&](const void *ptr, long ld, long stride) {
-    return (uintptr_t)ptr % 16 == 0 && ld % 4 == 0 && (d.batch == 1 || stride % 4 == 0);
-  };
-  const PackSide a{static_cast<const float *>(d.A), ws, d.M, d.lda, d.strideA, q.sa, !d.ta, vec(d.A, d.lda, d.strideA)};
-  const PackSide b{static_cast<const float *>(d.B), pb, d.N, d.ldb, d.strideB, q.sb, d.tb, vec(d.B, d.ldb, d.strideB)};
-  const int ya = (int)((d.M + 63) / 64), yb = (int)((d.N + 63) / 64);
+  const PackSide a{static_cast<const float *>(d.A), ws, d.M, d.lda, d.strideA, q.sa, !d.ta,
+                   vectors(d.A, d.lda, d.strideA, d.batch)};
+  const PackSide b{static_cast<const float *>(d.B), pb, d.N, d.ldb, d.strideB, q.sb, d.tb,
+                   vectors(d.B, d.ldb, d.strideB, d.batch)};
+  const int ya = (int)((d.M + 63) / 64), yb = plan.raw_b ? 0 : (int)((d.N + 63) / 64);
   hipLaunchKernelGGL(split_pack_kernel, dim3((unsigned)q.nkt, (unsigned)(ya + yb), (unsigned)d.batch), dim3(256), 0, s,
                      a, b, d.K, q.nkt, ya, gate, seq);
   if (hipError_t e = hipGetLastError()) return e;
   GemmParams p{};
   p.A = ws;
-  p.B = pb;
+  p.B = plan.raw_b ? d.B : pb;
+  p.ldb = d.ldb;
+  p.strideB = d.strideB;
   p.M = d.M;
   p.N = d.N;
   p.K = d.K;
@@ -361,7 +462,7 @@ hipError_t launch_split(const GemmDesc &d, const SplitPlan &plan, char *ws, floa
     p.alpha = 1.0f;
     p.act = -1;
   }
-  return launch_shape(plan.tile, p, q, d.batch, s);
+  return launch_shape(plan, plan.raw_b ? (d.tb ? 1 : 2) : 0, p, q, d.batch, s);
 }
 
 }  // namespace gn

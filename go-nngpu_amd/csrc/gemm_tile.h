@@ -243,5 +243,16 @@ __device__ __forceinline__ void sched_interleave() {
   if constexpr (NR > NP) __builtin_amdgcn_sched_group_barrier(0x100, NR - NP, 0);
 }
 
+// The same with up to VPM VALU instructions after every MFMA.
+template <int NM, int NR, int VPM = 5>
+__device__ __forceinline__ void sched_mix() {
+#pragma unroll
+  for (int g = 0; g < NM; ++g) {
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(0x002, VPM, 0);
+    if (g < NR) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+  }
+}
+
 }  // namespace
 }  // namespace gn

@@ -46,14 +46,18 @@ def _captured(fn):
     torch.cuda.synchronize()
 
 
-# (M, N, K): one round of 128 x 128 tiles; ragged rows, columns and K, split over K; two rounds of
+# (M, N, K), both operands packed: one round of 128 x 128 tiles; ragged rows, columns and K, split over K; two rounds of
 # 256 x 128 tiles; a K-tile count that its slices do not divide; K = 128 (four K-tiles).
 SHAPES = [(2048, 2048, 1024), (777, 1234, 4099), (4096, 4096, 512), (1100, 1100, 4000), (8192, 8192, 128),
           (2561, 2500, 2030)]
+# B split by the product kernel: 256-row and 128-row tiles, one launch and slices of K, ragged N, K of
+# whole K-tiles, with a remainder of whole vectors (NT's loads) and an odd one (NN; NT packs it)
+RAW_SHAPES = [(512, 11008, 1024), (512, 4096, 4096), (200, 1000, 2000), (160, 4100, 4132), (256, 5001, 2052),
+              (500, 3000, 1533)]
 
 
 @pytest.mark.parametrize("tA,tB", VARIANTS)
-@pytest.mark.parametrize("M,N,K", SHAPES)
+@pytest.mark.parametrize("M,N,K", SHAPES + RAW_SHAPES)
 def test_split_against_f64_and_the_fp32_cores(dev, M, N, K, tA, tB):
     import torch
 
@@ -76,7 +80,7 @@ def test_split_against_f64_and_the_fp32_cores(dev, M, N, K, tA, tB):
 
 
 @pytest.mark.parametrize("pads", [(0, 0, 0), (4, 8, 4), (1, 3, 5)])
-@pytest.mark.parametrize("M,N,K", [(2048, 2048, 1024), (777, 1234, 4099)])
+@pytest.mark.parametrize("M,N,K", [(2048, 2048, 1024), (777, 1234, 4099), (512, 11008, 1024), (512, 4096, 4096)])
 def test_split_epilogue_and_pitches(dev, M, N, K, pads):
     """alpha, beta over a prior C, bias and GELU, with leading dimensions wider than the rows
     (aligned to 16 bytes or not): C's padding stays, in one launch and over K slices."""
@@ -130,10 +134,11 @@ def test_split_parts_of_k_beyond_the_kept_scratch(dev):
     assert _rel(c, ref) <= 1e-6
 
 
-@pytest.mark.parametrize("M,N,K", [(2048, 2048, 1024), (777, 1234, 4099), (2050, 2046, 1030)])
+@pytest.mark.parametrize("M,N,K", [(2048, 2048, 1024), (777, 1234, 4099), (2050, 2046, 1030), (512, 11008, 1024), (512, 4096, 4096)])
 @pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan"), 3.4028234663852886e38, 2.0**36, -(2.0**40)])
+@pytest.mark.parametrize("beta", [0.0, 0.5])
 @pytest.mark.parametrize("side", ["a", "b"])
-def test_split_values_it_does_not_hold(dev, M, N, K, value, side):
+def test_split_values_it_does_not_hold(dev, M, N, K, value, side, beta):
     """One such value in either operand: the result is the fp32 matrix cores', with the
     infinities and NaN of the IEEE sums and nothing else touched."""
     import torch
@@ -146,10 +151,10 @@ def test_split_values_it_does_not_hold(dev, M, N, K, value, side):
     if side == "a":
         B[K - 1, 5] = 0.0  # infinity times zero: NaN in that column only
     c = torch.full((M, N), 7.0, device=dev)
-    G.gemm(A, B, c, beta=0.5)
+    G.gemm(A, B, c, beta=beta)
     c32 = torch.full((M, N), 7.0, device=dev)
-    _captured(lambda: G.gemm(A, B, c32, beta=0.5))
-    ref = A.double() @ B.double() + 3.5
+    _captured(lambda: G.gemm(A, B, c32, beta=beta))
+    ref = A.double() @ B.double() + 7.0 * beta
     fine = torch.isfinite(ref) & (ref.abs() < 3e38)
     rel = lambda x: float((x.double() - ref)[fine].norm() / ref[fine].norm())  # noqa: E731
     assert rel(c) <= max(1.5e-6, 1.5 * rel(c32))
