@@ -87,3 +87,24 @@ def test_linear_backward_full(dev, act):
     e = (O.rel_frob(dX.cpu().numpy(), rdX), O.rel_frob(dW.cpu().numpy(), rdW), O.rel_frob(gb.cpu().numpy(), rdb))
     _say("linear backward", act, e)
     assert max(e) <= 1e-5
+
+
+@pytest.mark.parametrize("chunks", [1, 2, 15, 16, 17, 31, 32, 47, 64])
+@pytest.mark.parametrize("cols", [1, 64, 130])
+def test_bias_sums_keep_their_order(dev, chunks, cols):
+    """Column sums are rows in order within a chunk, then chunks in order, in fp32: bit for bit
+    (rows / 8 chunks, rounded up, of equal length but for the last), at every remainder of the finishing kernel's groups of 16 chunks. The gradient is the
+    identity's with scale 1, so no product rounds."""
+    rng = np.random.default_rng(chunks * 1000 + cols)
+    rows = 8 * chunks - (3 if chunks > 1 else 0)  # the last chunk is short
+    dy = rng.standard_normal((rows, cols)).astype(np.float32)
+    _, gb = _act_bwd(dev, dy, dy, G.ACT_NONE)
+    want = np.zeros(cols, np.float32)
+    length = -(-rows // chunks)
+    for c in range(0, rows, length):
+        part = np.zeros(cols, np.float32)
+        for r in range(c, min(c + length, rows)):
+            part = part + dy[r]
+        want = want + part
+    _say("bias order", chunks, cols)
+    np.testing.assert_array_equal(gb, want)
