@@ -393,7 +393,11 @@ __device__ __forceinline__ void small_reduce_store(const GemmParams &p, float4_t
 // v_mfma_f32_16x16x4_f32 per s; fp16: E = 8, one v_mfma_f32_16x16x32_f16 per step), a
 // K-contiguous operand as one 16-byte vector when aligned. 64 elements of K are loaded before
 // their MFMAs run (a second register set that loads the next ones during the MFMAs measured
-// 10-20% slower: fewer waves fit). The KW partial tiles are added in LDS in wave order before
+// 10-20% slower: fewer waves fit). What bounds it is the latency of those load batches and the
+// instructions that address them, so whole K steps are loaded without bounds checks, from 32-bit
+// lane offsets that are computed once (rows past the product read its last one), and only a last,
+// partial step is masked: fp32 256 x 512 x 784 8.3 -> 5.8 us, 512^3 6.9 -> 5.8, fp16 100 x 130 x
+// 1000 NN 5.9 -> 3.7. The KW partial tiles are added in LDS in wave order before
 // the epilogue (small_reduce_store), so each element's summation order depends on K and KW
 // alone: the same for all four transpose layouts, aligned or not.
 // Per element type: the fragment vector V (E elements per lane and K step of KS elements)
@@ -417,7 +421,7 @@ struct SmallOps<_Float16> {
   }
 };
 
-template <typename T, int KW, int FM, int FN, bool TA, bool TB, bool VEC, int KB = 64>
+template <typename T, int KW, int FM, int FN, bool TA, bool TB, bool VEC, int KB>
 __global__ void __launch_bounds__(KW * 64) gemm_small_kernel(GemmParams p) {
   typedef SmallOps<T> Ops;
   typedef typename Ops::V V;
@@ -425,67 +429,118 @@ __global__ void __launch_bounds__(KW * 64) gemm_small_kernel(GemmParams p) {
   __shared__ float4_t red[KW][NF][64];
   const long m0 = (long)(blockIdx.x / p.tiles_n) * 16 * FM, n0 = (long)(blockIdx.x % p.tiles_n) * 16 * FN;
   const long z = blockIdx.z;
-  const T *A = static_cast<const T *>(p.A) + z * p.strideA;
-  const T *B = static_cast<const T *>(p.B) + z * p.strideB;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
-  const long steps = (p.K + KS - 1) / KS;
-  const long sb = steps * wave / KW, se = steps * (wave + 1) / KW;
+  const T *A = static_cast<const T *>(p.A) + z * p.strideA + (TA ? m0 : m0 * p.lda);
+  const T *B = static_cast<const T *>(p.B) + z * p.strideB + (TB ? n0 * p.ldb : n0);
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
+  const int steps = (int)((p.K + KS - 1) / KS), whole = (int)(p.K / KS);
+  const int sb = (int)((long)steps * wave / KW), se = (int)((long)steps * (wave + 1) / KW), fe = min(se, whole);
 
-  // One lane's E elements (k .. k + E - 1) of row r of op(A) or column r of op(B): rows past
-  // the product and k past K read as zero.
-  auto frag = [&](const T *X, long ld, bool kcontig, long r, bool rin, long k) {
-    V v;
+  // A lane's byte offset from a K step's start; rows past the product read the last one (what
+  // they give is not stored).
+  unsigned va[FM], vb[FN];
 #pragma unroll
-    for (int e = 0; e < E; ++e) v[e] = T(0);
-    if (!rin) return v;
+  for (int i = 0; i < FM; ++i) {
+    const unsigned r = (unsigned)min((long)(16 * i + li), p.M - 1 - m0);
+    va[i] = (unsigned)sizeof(T) * (TA ? r + E * lg * (unsigned)p.lda : r * (unsigned)p.lda + E * lg);
+  }
+#pragma unroll
+  for (int j = 0; j < FN; ++j) {
+    const unsigned c = (unsigned)min((long)(16 * j + li), p.N - 1 - n0);
+    vb[j] = (unsigned)sizeof(T) * (TB ? c * (unsigned)p.ldb + E * lg : c + E * lg * (unsigned)p.ldb);
+  }
+  auto at = [](const T *q, unsigned v0) { return reinterpret_cast<const T *>(reinterpret_cast<const char *>(q) + v0); };
+  // One lane's E elements of whole K step t.
+  auto frag = [&](const T *X, long ld, bool kcontig, unsigned v0, int t) {
+    V v;
     if (kcontig) {
-      const T *q = X + r * ld + k;
-      if (VEC) {  // K is a multiple of E: the E elements are all inside or all past K
-        if (k < p.K) v = *reinterpret_cast<const V *>(q);
+      const T *q = X + (long)t * KS;
+      if (VEC) {
+        v = *reinterpret_cast<const V *>(at(q, v0));
       } else {
 #pragma unroll
-        for (int e = 0; e < E; ++e)
-          if (k + e < p.K) v[e] = q[e];
+        for (int e = 0; e < E; ++e) v[e] = *at(q + e, v0);
       }
     } else {
 #pragma unroll
-      for (int e = 0; e < E; ++e)
-        if (k + e < p.K) v[e] = X[(k + e) * ld + r];
+      for (int e = 0; e < E; ++e) v[e] = *at(X + ((long)t * KS + e) * ld, v0);
     }
     return v;
   };
+  // The same of the last, partial K step: k past K counts as zero, read at the step's first k.
+  auto frag_end = [&](const T *X, long ld, bool kcontig, unsigned v0) {
+    V v;
+    const long k0 = (long)whole * KS;
+    const T *q = X + (kcontig ? k0 : k0 * ld);
+    const unsigned step = (unsigned)sizeof(T) * (kcontig ? 1u : (unsigned)ld), first = v0 - E * lg * step;
+    if (VEC && kcontig) {  // K is a multiple of E: the E elements are all inside or all past K
+      const bool in = k0 + E * lg < p.K;
+      v = *reinterpret_cast<const V *>(at(q, in ? v0 : first));
+#pragma unroll
+      for (int e = 0; e < E; ++e) v[e] = in ? v[e] : T(0);
+    } else {
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        const bool in = k0 + E * lg + e < p.K;
+        const T x = *at(q, in ? v0 + e * step : first);
+        v[e] = in ? x : T(0);
+      }
+    }
+    return v;
+  };
+  V ae[FM], be[FN];
+  if (se > fe) {  // used last, loaded first
+#pragma unroll
+    for (int i = 0; i < FM; ++i) ae[i] = frag_end(A, p.lda, !TA, va[i]);
+#pragma unroll
+    for (int j = 0; j < FN; ++j) be[j] = frag_end(B, p.ldb, TB, vb[j]);
+  }
 
   float4_t acc[FM][FN];
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
     for (int j = 0; j < FN; ++j) acc[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
-  for (long t0 = sb; t0 < se; t0 += U) {
+  auto multiply = [&](const V(&af)[FM], const V(&bf)[FN]) {
+#pragma unroll
+    for (int s = 0; s < Ops::MPS; ++s)
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) acc[i][j] = Ops::mma(af[i], bf[j], s, acc[i][j]);
+  };
+  auto batch = [&](int t0, auto part_c) {
+    constexpr bool PART = decltype(part_c)::value;  // fewer than U steps are left: the rest count as zeros
     V af[U][FM], bf[U][FN];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const bool live = t0 + u < se;
-      const long k = (t0 + u) * KS + E * lg;
+      const int t = PART ? min(t0 + u, fe - 1) : t0 + u;
 #pragma unroll
-      for (int i = 0; i < FM; ++i) {
-        const long r = m0 + 16 * i + li;
-        af[u][i] = frag(A, p.lda, !TA, r, live && r < p.M, k);
-      }
+      for (int i = 0; i < FM; ++i) af[u][i] = frag(A, p.lda, !TA, va[i], t);
 #pragma unroll
-      for (int j = 0; j < FN; ++j) {
-        const long c = n0 + 16 * j + li;
-        bf[u][j] = frag(B, p.ldb, TB, c, live && c < p.N, k);
-      }
+      for (int j = 0; j < FN; ++j) bf[u][j] = frag(B, p.ldb, TB, vb[j], t);
     }
+    __builtin_amdgcn_sched_barrier(0);  // all loads before the first MFMA
 #pragma unroll
-    for (int u = 0; u < U; ++u)
-#pragma unroll
-      for (int s = 0; s < Ops::MPS; ++s)
+    for (int u = 0; u < U; ++u) {
+      if (PART && u > 0) {
+        const bool live = t0 + u < fe;
 #pragma unroll
         for (int i = 0; i < FM; ++i)
 #pragma unroll
-          for (int j = 0; j < FN; ++j) acc[i][j] = Ops::mma(af[u][i], bf[u][j], s, acc[i][j]);
-  }
+          for (int e = 0; e < E; ++e) af[u][i][e] = live ? af[u][i][e] : T(0);
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+#pragma unroll
+          for (int e = 0; e < E; ++e) bf[u][j][e] = live ? bf[u][j][e] : T(0);
+      }
+      multiply(af[u], bf[u]);
+    }
+  };
+  int t0 = sb;
+  for (; t0 + U <= fe; t0 += U) batch(t0, std::false_type{});
+  if (t0 < fe) batch(t0, std::true_type{});
+  if (se > fe) multiply(ae, be);
   small_reduce_store<KW, FM, FN>(p, red, acc, m0, n0, z);
 }
 
@@ -1221,15 +1276,17 @@ hipError_t launch_small(GemmParams p, long batch, hipStream_t s) {
 }
 
 // The small-product kernel of shape code 100 KW + 10 FM + FN; hipErrorInvalidValue for
-// another code.
+// another code. Load batches of 64 elements of K; 48 for fp32 on 32 x 16 tiles, whose waves
+// hold few K steps (256 x 512 x 784: 5.8 us against 6.3 with 64; 128 for 16 waves took 16 x 16 x 4096 from
+// 13.3 to 15.3).
 template <typename T, bool TA, bool TB, bool VEC>
 hipError_t launch_small_code(int code, const GemmParams &p, long batch, hipStream_t s) {
   switch (code) {
     case 411: return launch_small<T, 4, 1, 1, TA, TB, VEC>(p, batch, s);
     case 811: return launch_small<T, 8, 1, 1, TA, TB, VEC>(p, batch, s);
     case 1611: return launch_small<T, 16, 1, 1, TA, TB, VEC>(p, batch, s);
+    case 421: return launch_small<T, 4, 2, 1, TA, TB, VEC, sizeof(T) == 4 ? 48 : 64>(p, batch, s);
     case 422: return launch_small<T, 4, 2, 2, TA, TB, VEC>(p, batch, s);
-    case 822: return launch_small<T, 8, 2, 2, TA, TB, VEC>(p, batch, s);
     default: return hipErrorInvalidValue;
   }
 }
@@ -1372,28 +1429,45 @@ inline int skinny_tile(long M, long N, long K, long batch, bool f16, bool ta, bo
   return t16 * 16 <= 4096 ? 1611 : t16 * 8 <= 4096 ? 811 : 411;
 }
 
+// The small-product kernel's 32-bit offsets reach 31 rows past the tile's first.
+inline bool small_offsets_fit(long lda, long ldb) { return lda <= (1L << 24) && ldb <= (1L << 24); }
+
+// Its workgroup tile (10 FM + FN): 16 x 16 while that makes at most one workgroup per CU, 32 x
+// 16 while that does, 16 x 16 again up to two per CU, else 32 x 32 (16 x 16 / 32 x 16 / 32 x 32,
+// four waves: fp32 256 x 512 x 784 7.0 / 5.8 / 8.3 us, 512^3 8.0 / 7.2 / 5.8; fp16 5.1 / 4.2 /
+// 4.4 and 5.9 / 5.0 / 4.0; fp32 200 x 600 x 600, 266 tiles of 32 x 16, 7.0 / 8.1).
+inline int small_shape(long M, long N, long batch) {
+  const long n16 = (N + 15) / 16 * batch, t16 = (M + 15) / 16 * n16;
+  return t16 <= 256 ? 11 : (M + 31) / 32 * n16 <= 256 ? 21 : t16 <= 512 ? 11 : 22;
+}
+
 // The small-product kernel's shape for an fp16 product (100 KW + 10 FM + FN), or 0 for the
-// tiled kernels. fp16 MFMAs are 8x the fp32 rate, so the 64 x 64 register-staged kernel stays
-// ahead from fewer tiles than in fp32: the small kernel is taken for at most 16 of them, for
-// K up to 1024 or below 2^24 multiply-adds in all (no split-K there), always with 16 x 16
-// workgroup tiles and 16 waves from 24 32-element K steps (K > 736), 8 from 8 (K > 224), else
-// 4: with fp16 a wave's K step is one MFMA, and more waves with fewer steps each measured
-// faster. Kernel times on MI355X (rocprofv3 kernel trace), tiled -> small, NN: 256^3 5.70 ->
-// 4.47 us; 100 x 130 x 1000 30.9 -> 9.5 us; 64 x 128 x 784 9.0 -> 6.1 us; 256^2 x 1024 10.2
-// -> 6.9 us; 16 x 16 x 4096 29.1 -> 12.8 us. 384^2 and larger, and 64^2 x 4096, stay on the
-// tiled kernels (4.5 against 4.6 us at 384^2 x 64, 11.9 against 13.9 us at 64^2 x 4096).
-inline int f16_small_tile(long M, long N, long K, long batch, bool ta, bool tb) {
+// tiled kernels. Times of a call, tiled -> small, NN and NT: 512^3 (64 tiles of 64 x 64) 6.9 ->
+// 4.0 and 4.4 us, 512^2 x 2048 12.3 -> 7.9 and 9.5, 640^2 x 1024 (100 tiles) 11.1 -> 8.0 and
+// 9.7; 768^2 x 512 (144 tiles) 7.1 -> 6.9 and 8.1. So it is taken for at most 64 such tiles and
+// K up to 2048, 100 and K up to 1024 if the operands are aligned (`vec`), and for few
+// multiply-adds (no split-K there) on at most 16; unaligned on at most 16 tiles and K up to 1024,
+// and TN, where neither operand's elements of K lie together, up to 1024 too (24 x 3000 x 2048:
+// 19.9 us against 10.6).
+// 16 x 16 tiles split K over 16 waves from 96 32-element K steps, 8 from 8, else 4: 64 x 128 x
+// 1000 takes 3.8 / 3.6 / 3.7 us with 4 / 8 / 16.
+inline int f16_small_tile(long M, long N, long K, long batch, bool ta, bool tb, bool vec) {
   if (const int c = skinny_tile(M, N, K, batch, true, ta, tb)) return c;
   const long tiles64 = ((M + 63) / 64) * ((N + 63) / 64) * batch;
-  if (tiles64 > 16) return 0;
-  if (!(K <= 1024 || (double)M * N * K * batch < (double)(1L << 24))) return 0;
+  const bool few_macs = (double)M * N * K * batch < (double)(1L << 24);
+  if (!(tiles64 <= 16 && (K <= 1024 || few_macs)) &&
+      !(vec && ((tiles64 <= 64 && K <= (ta && !tb ? 1024 : 2048)) || (tiles64 <= 100 && K <= 1024))))
+    return 0;
   const long steps = (K + 31) / 32;
-  return steps >= 24 ? 1611 : steps >= 8 ? 811 : 411;
+  const int shape = small_shape(M, N, batch);
+  return shape != 11 ? 400 + shape : steps >= 96 ? 1611 : steps >= 8 ? 811 : 411;
 }
 
 template <bool TA, bool TB, bool VEC>
 hipError_t pick_f16(const GemmParams &p, long batch, hipStream_t s) {
-  if (const int code = f16_small_tile(p.M, p.N, p.K, batch, TA, TB)) return launch_small_code<_Float16, TA, TB, VEC>(code, p, batch, s);
+  if (small_offsets_fit(p.lda, p.ldb))
+    if (const int code = f16_small_tile(p.M, p.N, p.K, batch, TA, TB, VEC))
+      return launch_small_code<_Float16, TA, TB, VEC>(code, p, batch, s);
   if constexpr (!VEC) {
     // Unaligned shapes take the element-wise load path on the smallest tile only.
     return launch_f16<64, 64, 64, 2, 2, TA, TB, VEC>(p, batch, s);
@@ -1482,37 +1556,35 @@ hipError_t launch_f32_ring_best(const GemmParams &p, long batch, hipStream_t s) 
 
 // The small-product kernel's shape for an fp32 product, as 100 KW + 10 FM + FN, or 0 for the
 // tiled kernels. It is taken while the 64 x 64 tiles would leave at least three quarters of
-// the CUs idle (at most 64 tiles), for K up to 1024, for K up to 4096 at 4 tiles or fewer,
-// and for any K below 2^24 multiply-adds in all (where the tiled path has no split-K).
-// Workgroups of 16 x 16 tiles while there are at most 256 of them (or K is at most 32), or at
-// most 512 with K over 272; 32 x 32 beyond (128 x 784 x 784: 8.4 us on 16 x 16 tiles against
-// 10.2 on 32 x 32; 256 x 512 x 256: 7.3 against 6.6). As many K-splitting waves (4, 8, or 16
-// with 16 x 16 tiles) as leave each wave at least three 16-element K steps and the grid at most
-// 2048 waves. Kernel times on MI355X (rocprofv3 kernel trace), tiled -> small: 256^3 7.7 -> 4.2
-// us; 128 x 784 x 784 21.5 -> 8.4 us; 100 x 130 x 1000 49.7 -> 10.6 us; 512^2 x 1024 16.3 ->
-// 11.1 us; 16 x 16 x 4096 66.3 -> 13.6 us. At 768^2 (144 tiles), at 256^2 x 4096 and at 64^2 x
-// 16384 the tiled path (split-K for the long K) is as fast or faster.
+// the CUs idle (at most 64 tiles) for K up to 1024, on at most 36 tiles for K up to 1536, 16 for
+// 2048, 4 for 4096, and for any K below 2^24 multiply-adds in all (where the tiled path has no
+// split-K). Times of a call, tiled -> small, NN and NT: 384^2 x 1536 15.5 -> 11.3 and 13.5 us;
+// 256^2 x 2048 11.4 -> 7.5 and 9.6; 512^2 x 2048 (64 tiles) 17.2 -> 16.0 and 18.0; 768^2 x 512
+// (144 tiles) 11.6 -> 14.7 and 15.2. 32 x 16 tiles also below 12 16-element K steps, where 32 x
+// 32 ones leave the waves little to do (512^2 x 128: 4.1 against 4.5 us), 16 x 16 up to 2 steps.
+// Four waves split K; on 16 x 16 tiles 8 from 96 steps and 16 from 256 (up to 1024
+// waves in all): level there (256^2 x 2048: 7.5 / 7.9 / 8.6 us with 4 / 8 / 16; 64 x 128 x 1000: 4.4 /
+// 5.3 / 5.7) and their sums are shorter.
 inline int f32_small_tile(long M, long N, long K, long batch, bool ta, bool tb) {
   if (const int c = skinny_tile(M, N, K, batch, false, ta, tb)) return c;
   const long tiles64 = ((M + 63) / 64) * ((N + 63) / 64) * batch;
   if (tiles64 > 64) return 0;
   const bool few_macs = (double)M * N * K * batch < (double)(1L << 24);
-  if (!(K <= 1024 || (tiles64 <= 4 && K <= 4096) || few_macs)) return 0;
+  const long most = tiles64 <= 4 ? 4096 : tiles64 <= 16 ? 2048 : tiles64 <= 36 ? 1536 : 1024;
+  if (K > most && !few_macs) return 0;
   const long t16 = ((M + 15) / 16) * ((N + 15) / 16) * batch, steps = (K + 15) / 16;
-  const bool f11 = t16 <= 256 || steps <= 2 || (t16 <= 512 && steps >= 18);
-  const long wgs = f11 ? t16 : (t16 + 3) / 4;
-  int kw = 4;
-  for (int c : {16, 8}) {
-    if ((c == 16 && !f11) || 3 * c > steps || wgs * c > 2048) continue;
-    kw = c;
-    break;
-  }
-  return kw * 100 + (f11 ? 11 : 22);
+  int shape = small_shape(M, N, batch);
+  if (steps <= 2) shape = 11;
+  else if (steps < 12 && shape == 22) shape = 21;
+  if (shape != 11 || steps < 96) return 400 + shape;
+  return steps >= 256 && t16 * 16 <= 1024 ? 1611 : 811;
 }
 
 template <bool TA, bool TB, bool VEC>
 hipError_t pick_f32(const GemmParams &p, long batch, hipStream_t s) {
-  if (const int code = f32_small_tile(p.M, p.N, p.K, batch, TA, TB)) return launch_small_code<float, TA, TB, VEC>(code, p, batch, s);
+  if (small_offsets_fit(p.lda, p.ldb))
+    if (const int code = f32_small_tile(p.M, p.N, p.K, batch, TA, TB))
+      return launch_small_code<float, TA, TB, VEC>(code, p, batch, s);
   if constexpr (!VEC) {
     return launch_f32<64, 64, 16, 2, 2, TA, TB, VEC>(p, batch, s);
   } else {
@@ -1870,19 +1942,22 @@ hipError_t dispatch_behind(bool ta, bool tb, const GemmParams &p, long batch, hi
   return tb ? launch_f32_behind<false, true, VEC>(p, batch, s) : launch_f32_behind<false, false, VEC>(p, batch, s);
 }
 
-// Where gemm_rows.hip takes a product it can (plan_rows): always up to 16 rows; up to 32 from 2^20
-// elements of W, in fp16 below 2^25 (28 rows x 11008 x 4096: 28.9 us against 27.7 on the split-K
-// ring); up to 64 in fp16 from 2^20 to 12 M elements (64 x 4096 x 1024: 12.7 -> 7.9 us; at 16 M
-// level, at 45 M 36 against 30), in fp32 by price (the fp32 tiles' is for a
+// Where gemm_rows.hip takes a product it can (plan_rows). Up to 16 rows: always, but for what the
+// small-product kernel takes with W below 2^20 elements (1 x 1000 x 1000 fp16 3.8 us against 2.9
+// there). Up to 32 from 2^20 elements of W, in fp16 below 2^25 (28 rows x 11008 x 4096: 28.9 us
+// against 27.7 on the split-K ring); up to 64 in fp16 from 2^20 to 12 M elements (at 16 M level,
+// at 45 M 36 against 30), both fp16 ones only past the small-product kernel's range (64 x 1024 x
+// 1024: 7.2 us against 4.5), in fp32 by price (the fp32 tiles' is for a
 // warm W and 15% low with W from HBM: 40 x 11008 x 4096 74 -> 59), and instead of the small-product
-// kernel for K of 2048 and more (64 x 256 x 4096: 17.2 -> 11.3 us; 64 x 512 x 512: 8.1 against 5.0).
+// kernel for K of 2048 and more (32 x 2048 x 1024: 7.4 us against 5.3; 64 x 256 x 4096: 17.2 -> 11.3 us; 64 x 512 x 512: 8.1 against 5.0).
 bool takes_rows(const GemmDesc &d, const RowsPlan &rows, bool a_ok, bool b_ok, bool small) {
-  if (d.M <= 16) return true;
   const double w = (double)d.N * (double)d.K;
+  if (small && w < (double)(1L << 20)) return false;
+  if (d.M <= 16) return true;
   if (w < (double)(1L << 20)) return false;
-  if (d.dtype == GN_F16) return w < (d.M <= 32 ? (double)(1L << 25) : 12.0e6);
-  if (d.M <= 32) return true;
-  return small ? d.K >= 2048 : rows.us < 1.15 * (f32_cores_us(d, a_ok, b_ok) + 3.0);
+  if (d.dtype == GN_F16) return !small && w < (d.M <= 32 ? (double)(1L << 25) : 12.0e6);
+  if (small) return d.K >= 2048;
+  return d.M <= 32 || rows.us < 1.15 * (f32_cores_us(d, a_ok, b_ok) + 3.0);
 }
 
 // How a product runs through launch_split within the scratch a stream keeps: nb batches and kc
@@ -2030,8 +2105,9 @@ int launch_gemm(const GemmDesc &d, hipStream_t s, CError *err) {
         (size_t)((a_ok ? 0 : d.M) + (b_ok ? 0 : d.N)) * (size_t)Kp * esz * (size_t)std::min(kMaxZ, d.batch);
     const bool big = (double)d.M * d.N * d.K >= (double)(1L << 24);
     const long pack_grid_y = (a_ok ? 0 : (d.M + 63) / 64) + (b_ok ? 0 : (d.N + 63) / 64);
-    const bool small = (d.dtype == GN_F32 ? f32_small_tile(d.M, d.N, d.K, d.batch, d.ta, d.tb)
-                                          : f16_small_tile(d.M, d.N, d.K, d.batch, d.ta, d.tb)) != 0;
+    const bool small = small_offsets_fit(d.lda, d.ldb) &&
+                       (d.dtype == GN_F32 ? f32_small_tile(d.M, d.N, d.K, d.batch, d.ta, d.tb)
+                                          : f16_small_tile(d.M, d.N, d.K, d.batch, d.ta, d.tb, vec)) != 0;
     bool pack = !vec && big && !small && pack_bytes <= ((size_t)4 << 30) && pack_grid_y <= 65535;
     // A product of at most 64 rows (takes_rows), slices of K only outside graph capture (their
     // partial products take scratch) and where the scratch can be had.
