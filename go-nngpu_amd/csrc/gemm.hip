@@ -7,7 +7,9 @@
 // kernels (metal_bridge_kernels.m:28-110) and the fused_linear_activation kernel
 // (default.metal:459-509).
 //
-// Two kernel families share the epilogue and the tile order: the DMA-ring kernels
+// Large fp32 products run on the bf16 matrix cores (gemm_split.hip), products of at most 64 rows
+// on kernels that stream W (gemm_rows.hip), and the smallest on gemm_small_kernel. For the rest
+// two kernel families share the epilogue and the tile order: the DMA-ring kernels
 // gemm_f16_ring_kernel and gemm_f32_ring_kernel (large fp16 and fp32 problems; described
 // at their definitions; gemm_f16_ring_mf32_kernel is the NN 256 x 256 ring on 32 x 32 x 16
 // instructions, kept for measurement behind GONNGPU_F16_MFMA32=1) and the register-staged
@@ -396,7 +398,7 @@ __device__ __forceinline__ void small_reduce_store(const GemmParams &p, float4_t
 // 10-20% slower: fewer waves fit). What bounds it is the latency of those load batches and the
 // instructions that address them, so whole K steps are loaded without bounds checks, from 32-bit
 // lane offsets that are computed once (rows past the product read its last one), and only a last,
-// partial step is masked: fp32 256 x 512 x 784 8.3 -> 5.8 us, 512^3 6.9 -> 5.8, fp16 100 x 130 x
+// partial step is masked: fp32 256 x 512 x 784 8.3 -> 5.8 us, 512^3 6.9 -> 5.8, fp16 100 x 136 x
 // 1000 NN 5.9 -> 3.7. The KW partial tiles are added in LDS in wave order before
 // the epilogue (small_reduce_store), so each element's summation order depends on K and KW
 // alone: the same for all four transpose layouts, aligned or not.
@@ -1435,7 +1437,7 @@ inline bool small_offsets_fit(long lda, long ldb) { return lda <= (1L << 24) && 
 // Its workgroup tile (10 FM + FN): 16 x 16 while that makes at most one workgroup per CU, 32 x
 // 16 while that does, 16 x 16 again up to two per CU, else 32 x 32 (16 x 16 / 32 x 16 / 32 x 32,
 // four waves: fp32 256 x 512 x 784 7.0 / 5.8 / 8.3 us, 512^3 8.0 / 7.2 / 5.8; fp16 5.1 / 4.2 /
-// 4.4 and 5.9 / 5.0 / 4.0; fp32 200 x 600 x 600, 266 tiles of 32 x 16, 7.0 / 8.1).
+// 4.4 and 5.9 / 5.0 / 4.0; fp32 200 x 600 x 600, 266 tiles of 32 x 16, 6.6 / 8.1).
 inline int small_shape(long M, long N, long batch) {
   const long n16 = (N + 15) / 16 * batch, t16 = (M + 15) / 16 * n16;
   return t16 <= 256 ? 11 : (M + 31) / 32 * n16 <= 256 ? 21 : t16 <= 512 ? 11 : 22;
@@ -1949,7 +1951,7 @@ hipError_t dispatch_behind(bool ta, bool tb, const GemmParams &p, long batch, hi
 // at 45 M 36 against 30), both fp16 ones only past the small-product kernel's range (64 x 1024 x
 // 1024: 7.2 us against 4.5), in fp32 by price (the fp32 tiles' is for a
 // warm W and 15% low with W from HBM: 40 x 11008 x 4096 74 -> 59), and instead of the small-product
-// kernel for K of 2048 and more (32 x 2048 x 1024: 7.4 us against 5.3; 64 x 256 x 4096: 17.2 -> 11.3 us; 64 x 512 x 512: 8.1 against 5.0).
+// kernel for K of 2048 and more (32 x 2048 x 1024: 7.4 us against 5.2; 64 x 256 x 4096: 17.2 -> 11.3 us; 64 x 512 x 512: 8.1 against 5.0).
 bool takes_rows(const GemmDesc &d, const RowsPlan &rows, bool a_ok, bool b_ok, bool small) {
   const double w = (double)d.N * (double)d.K;
   if (small && w < (double)(1L << 20)) return false;

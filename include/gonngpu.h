@@ -311,16 +311,20 @@ int gn_synchronize(void *stream, CError *err);
 /* General GEMM on device pointers:
  *   C[M,N] = act( alpha * op(A) * op(B) + beta * C + bias[n] )
  * op(A) is A[M,K] (lda >= K) or, with transA, A stored [K,M] (lda >= M); likewise B.
- * dtype GN_F32: A, B fp32, fp32 MFMA (v_mfma_f32_16x16x4_f32).
+ * dtype GN_F32: A, B fp32, on v_mfma_f32_16x16x4_f32 or, for large products, as exact sums of
+ * three bf16 parts on the bf16 MFMA with fp32 accumulation (no larger error; operands with
+ * infinities, NaN or magnitudes of 2^36 and above take the fp32 MFMA).
  * dtype GN_F16: A, B fp16, fp32 accumulate (v_mfma_f32_16x16x32_f16).
  * C and bias are fp32; bias may be NULL; beta == 0 never reads C.
  * batch >= 1 with element strides strideA/B/C between consecutive problems.
- * Outside HIP graph capture two paths use a scratch block that the library keeps per stream
- * (grown on demand from its pool): operands whose pointer, leading dimension or row length
+ * Outside HIP graph capture four paths use a scratch block that the library keeps per stream
+ * (grown on demand from its pool): large fp32 products (their parts), products of at most 64
+ * rows that are summed over slices of K, operands whose pointer, leading dimension or row length
  * is not a multiple of 16 bytes, in products of at least 2^24 multiply-adds, are first
  * copied into padded K-contiguous buffers, and batch-1 products with few output tiles and a
  * long K are summed over slices of K (partial products, then a reduce in slice order).
- * Under capture neither is taken, and nothing is allocated.
+ * Under capture none is taken, and nothing is allocated. Where the scratch cannot be had, the
+ * first two run without it.
  * Codes: -1 invalid argument, -3 scratch allocation failed, -6 launch error. */
 int gn_gemm(int dtype, int transA, int transB, long M, long N, long K, float alpha, const void *A, long lda,
             long strideA, const void *B, long ldb, long strideB, float beta, float *C, long ldc, long strideC,
