@@ -1962,53 +1962,6 @@ bool takes_rows(const GemmDesc &d, const RowsPlan &rows, bool a_ok, bool b_ok, b
   return d.M <= 32 || rows.us < 1.15 * (f32_cores_us(d, a_ok, b_ok) + 3.0);
 }
 
-// How a product runs through launch_split within the scratch a stream keeps: nb batches and kc
-// of K at a time (a multiple of 32; later parts of K add to C), each by `plan`.
-struct SplitCut {
-  long nb = 0, kc = 0;
-  SplitPlan plan;
-  size_t ws_bytes = 0;
-};
-
-// true when the product runs on the bf16 matrix cores: priced (the operands' packing, the
-// product, the reduce, 3 us for the fp32 kernels that stand behind it) at least 7% below the
-// fp32 matrix cores. Both prices were checked on 44 shapes (device times, fp32 -> bf16 parts, us):
-// taken 2048 x 2048 x 512 35 -> 35, 4096 x 4096 x 256 73 -> 60, 777 x 1234 x 4099 106 -> 74, 512 x
-// 11008 x 4096 369 -> 332, 2560^3 271 -> 167, 4096^3 928 -> 606; left on the fp32 cores, where the
-// packing or the fixed 15 us weigh too much: 1024^3 21 -> 35, 1280^3 42 -> 42, 256 x 4096 x 4096 71
-// -> 82, 128 x 8192 x 8192 139 -> 255. None of the 44 got slower; of those left, 512 x 4096 x 4096
-// would have gained most (125 -> 114).
-bool cut_split(const GemmDesc &d, bool a_ok, bool b_ok, SplitCut *cut) {
-  constexpr size_t kLimit = kScratchRetainBytes - 512;  // less the gate's block and the partials' rounding up
-  GemmDesc q = d;
-  if (!plan_split(q, &cut->plan)) return false;
-  double us = cut->plan.us;
-  size_t bytes = cut->plan.pack_bytes + cut->plan.part_bytes;
-  if (bytes > kLimit && d.batch > 1) {
-    q.batch = std::max(1L, (long)((double)kLimit / (double)bytes * (double)d.batch));
-    if (!plan_split(q, &cut->plan)) return false;
-    us = cut->plan.us * (double)d.batch / (double)q.batch;
-    bytes = cut->plan.pack_bytes + cut->plan.part_bytes;
-  }
-  if (bytes > kLimit) {
-    if (d.batch > 1) return false;
-    const long parts = (long)(bytes / kLimit) + 1;
-    q.K = ((d.K + parts - 1) / parts + 31) / 32 * 32;
-    q.beta = 1.0f;
-    if (q.K < 1024 || !plan_split(q, &cut->plan)) return false;
-    if (cut->plan.raw_b && d.K % 4) return false;  // the last part's K is not the planned one
-    us = (double)parts * cut->plan.us + (double)(parts - 1) * 8.0 * (double)d.M * d.N / 5.0e6;
-    bytes = cut->plan.pack_bytes + cut->plan.part_bytes;
-    if (bytes > kLimit) return false;
-  }
-  cut->nb = q.batch;
-  cut->kc = q.K;
-  cut->ws_bytes = bytes + 512;
-  // (the fp32 tiles' prices are for operands in the caches: with B from HBM the tiles of a few row
-  // blocks, where a raw B is the choice, took 15-30% more)
-  return us + 3.0 < (cut->plan.raw_b ? 1.0 : 0.93) * f32_cores_us(d, a_ok, b_ok);
-}
-
 // Enqueues the product by `cut` with ws (cut.ws_bytes) as its workspace. Behind every part the
 // fp32 kernels are enqueued too; they return at once unless an operand holds a value the split
 // does not (an infinity, a NaN, or 2^36 and more), in which case the part's split kernels wrote
@@ -2029,7 +1982,7 @@ hipError_t run_split(const GemmDesc &d, const SplitCut &cut, bool vec, char *ws,
       if (k > 0) q.beta = 1.0f;
       if (k + cut.kc < d.K) q.bias = nullptr, q.act = -1;
       SplitPlan plan = cut.plan;
-      plan.S = (int)std::min<long>(plan.S, (q.K + 31) / 32);
+      plan.S = split_slices(plan, q.K);
       // a value no earlier call left in *gate; a chance match in fresh scratch only costs time
       const unsigned long long seq = ++calls;
       if (hipError_t e = launch_split(q, plan, packed, part, gate, seq, s)) return e;
@@ -2049,6 +2002,43 @@ hipError_t run_split(const GemmDesc &d, const SplitCut &cut, bool vec, char *ws,
 }
 
 }  // namespace
+
+// true when the product runs on the bf16 matrix cores: priced (the operands' packing, the
+// product, the reduce, 3 us for the fp32 kernels that stand behind it) at least 7% below the
+// fp32 matrix cores. Both prices were checked on 44 shapes (device times, fp32 -> bf16 parts, us):
+// taken 2048 x 2048 x 512 35 -> 35, 4096 x 4096 x 256 73 -> 60, 777 x 1234 x 4099 106 -> 74, 512 x
+// 11008 x 4096 369 -> 332, 2560^3 271 -> 167, 4096^3 928 -> 606; left on the fp32 cores, where the
+// packing or the fixed 15 us weigh too much: 1024^3 21 -> 35, 1280^3 42 -> 42, 256 x 4096 x 4096 71
+// -> 82, 128 x 8192 x 8192 139 -> 255. None of the 44 got slower; of those left, 512 x 4096 x 4096
+// would have gained most (125 -> 114).
+bool cut_split(const GemmDesc &d, bool a_ok, bool b_ok, SplitCut *cut) {
+  constexpr size_t kLimit = kScratchRetainBytes - 512;  // less the gate's block and the partials' rounding up
+  long nb = d.batch, kc = d.K;
+  if (!plan_split(d, nb, kc, &cut->plan)) return false;
+  double us = cut->plan.us;
+  size_t bytes = cut->plan.pack_bytes + cut->plan.part_bytes;
+  if (bytes > kLimit && d.batch > 1) {
+    nb = std::max(1L, (long)((double)kLimit / (double)bytes * (double)d.batch));
+    if (!plan_split(d, nb, kc, &cut->plan)) return false;
+    us = cut->plan.us * (double)d.batch / (double)nb;
+    bytes = cut->plan.pack_bytes + cut->plan.part_bytes;
+  }
+  if (bytes > kLimit) {
+    if (d.batch > 1) return false;
+    const long parts = (long)(bytes / kLimit) + 1;
+    kc = ((d.K + parts - 1) / parts + 31) / 32 * 32;
+    if (kc < 1024 || !plan_split(d, nb, kc, &cut->plan)) return false;
+    us = (double)parts * cut->plan.us + (double)(parts - 1) * 8.0 * (double)d.M * d.N / 5.0e6;
+    bytes = cut->plan.pack_bytes + cut->plan.part_bytes;
+    if (bytes > kLimit) return false;
+  }
+  cut->nb = nb;
+  cut->kc = kc;
+  cut->ws_bytes = bytes + 512;
+  // (the fp32 tiles' prices are for operands in the caches: with B from HBM the tiles of a few row
+  // blocks, where a raw B is the choice, took 15-30% more)
+  return us + 3.0 < (cut->plan.raw_b ? 1.0 : 0.93) * f32_cores_us(d, a_ok, b_ok);
+}
 
 bool act_supported(int act) { return act == -1 || act == 0 || act == 1 || act == 2 || (act >= 4 && act <= 7); }
 

@@ -12,17 +12,36 @@ constexpr float kSplitMax = 68719476736.0f;  // 2^36
 constexpr int kSplitBlock = 3072;            // bytes of 16 rows x 32 k in three bf16 parts
 constexpr long kSplitMaxK = 1L << 20;        // K up to which no partial sum overflows
 
-// How a product of `batch` M x N x K problems is cut: tile (index into the kernel's shapes), S
-// slices of K, the device time it is priced at (us, pack and reduce included), and the bytes
-// of the packed operands and the partial products.
+// How one launch of a product runs: tile (index into the kernel's shapes), S slices of K, the
+// device time it is priced at (us, pack and reduce included), and the bytes of the packed
+// operands and the partial products.
 struct SplitPlan {
   int tile = 0, S = 1;
   bool raw_b = false;  // B is split by the product kernel instead of packed
   double us = 0;
   size_t pack_bytes = 0, part_bytes = 0;
 };
-// false: a shape the split kernels do not take.
-bool plan_split(const GemmDesc &d, SplitPlan *out);
+// The plan for the parts of d that a launch takes: nb of its batches and kc of its K (a multiple
+// of 32, or all of K; parts of K add to C). It holds for every part: alignments are those of any
+// batch's and any part's operands, and the last part may be shorter. false: a shape the split
+// kernels do not take.
+bool plan_split(const GemmDesc &d, long nb, long kc, SplitPlan *out);
+// The slices of a part with K `k` by that plan: none is empty.
+inline int split_slices(const SplitPlan &plan, long k) {
+  const long nkt = (k + 31) / 32;
+  return plan.S < nkt ? plan.S : (int)nkt;
+}
+
+// How a product runs through launch_split within the scratch a stream keeps: nb batches and kc
+// of K at a time, each by `plan`.
+struct SplitCut {
+  long nb = 0, kc = 0;
+  SplitPlan plan;
+  size_t ws_bytes = 0;
+};
+// true when the product runs on the bf16 matrix cores (gemm.hip). a_ok, b_ok: the operand suits
+// the aligned fp32 kernels.
+bool cut_split(const GemmDesc &d, bool a_ok, bool b_ok, SplitCut *cut);
 // The partials' stride in floats: M x N rounded up to a multiple of 4.
 inline long splitk_stride(long M, long N) { return (M * N + 3) / 4 * 4; }
 

@@ -376,9 +376,10 @@ bool vectors(const void *ptr, long ld, long stride, long batch) {
 
 }  // namespace
 
-bool plan_split(const GemmDesc &d, SplitPlan *out) {
-  const long M = d.M, N = d.N, K = d.K, batch = d.batch, nkt = (K + 31) / 32;
-  const bool beta = d.beta != 0.0f;
+bool plan_split(const GemmDesc &d, long nb, long kc, SplitPlan *out) {
+  const long M = d.M, N = d.N, K = kc, batch = nb, nkt = (K + 31) / 32;
+  const bool beta = d.beta != 0.0f || kc < d.K;
+  const long last_k = d.K - (d.K - 1) / kc * kc;  // of the last part
   if (K < 32 || K > kSplitMaxK || batch > 16384 || (M + 63) / 64 + (N + 63) / 64 > 65535) return false;
   const size_t pa = (size_t)blocks16(M) * nkt * kSplitBlock, pb = (size_t)blocks16(N) * nkt * kSplitBlock;
   if (pa >= ring::kNumRecords) return false;  // 32-bit copy offsets
@@ -388,8 +389,9 @@ bool plan_split(const GemmDesc &d, SplitPlan *out) {
   // power, and the reduce. Slices keep at least 8 K-tiles. A raw B saves its packing (10 bytes per
   // element) and costs a 256-row tile's K-tile about a tenth, a 128-row tile's half as much again: it
   // pays for up to about 512 rows (512 x 11008 x 4096 NT 323 -> 250 us, 256 rows 217 -> 156; 1024 x 4096 x
-  // 1024: level). It reads 16-byte vectors of a K-contiguous B.
-  const bool raw_ok = d.tb ? vectors(d.B, d.ldb, d.strideB, batch) && K % 4 == 0 : true;
+  // 1024: level). It reads 16-byte vectors of a K-contiguous B, in every batch and part (kc is a
+  // multiple of 32, or K).
+  const bool raw_ok = d.tb ? vectors(d.B, d.ldb, d.strideB, d.batch) && d.K % 4 == 0 : true;
   out->us = 1e30;
   for (int form = 0; form < 4; ++form) {
     const int tile = form & 1;
@@ -402,7 +404,8 @@ bool plan_split(const GemmDesc &d, SplitPlan *out) {
     if (tiles > (1L << 30)) return false;
     for (long S = 1; S <= (batch == 1 ? 32 : 1) && S <= nkt; ++S) {
       if (S > 1 && nkt / S < 8) break;
-      if (raw && S == 1 && beta) continue;
+      // a raw B without slices writes C before its values are known: not where C counts, in any part
+      if (raw && beta && std::min(S, (last_k + 31) / 32) == 1) continue;
       const long w = tiles * S, rounds = (w + 255) / 256;
       const double kt = (double)((nkt + S - 1) / S), busy = (double)w / (256.0 * (double)rounds);
       const double wg = raw ? (tile == 0 ? 10.0 + (1.75 + 0.6 * busy) * kt : 8.0 + 1.36 * kt)

@@ -114,6 +114,40 @@ def test_split_batched(dev):
         assert _rel(c[i], A[i].double() @ B[i].double().t().contiguous()) <= 5e-7
 
 
+# M, N, K, batch, layout, elements between the batches' B, form: parts of several batches or of a single one, or of
+# K; "raw": B split by the product kernel (test_split_plan.py checks that each case is cut so)
+CUTS = [(512, 1024, 4096, 48, "nn", 0, "batch-raw"), (400, 4096, 4096, 6, "nt", 1, "batch"),
+        (512, 1000, 100000, 2, "nt", 0, "single-raw"), (512, 1000, 100000, 2, "nt", 4, "single-raw"),
+        (512, 11008, 4096, 2, "nt", 1, "single"), (500, 1000, 200004, 1, "nt", 0, "k-raw"),
+        (500, 1000, 200001, 1, "nn", 0, "k-raw")]
+
+
+@pytest.mark.parametrize("M,N,K,batch,layout,gap,form", CUTS)
+def test_split_cut_into_parts(dev, M, N, K, batch, layout, gap, form):
+    """A batch cut into launches of several batches or of one, with batch strides that keep the rows
+    of a K-contiguous B on 16 bytes or not, and K cut into parts with a raw B."""
+    import torch
+
+    g = torch.Generator(device=dev).manual_seed(M + N + gap)
+    A = torch.randn((batch, M, K), generator=g, device=dev)
+    stride = N * K + gap
+    flat = torch.randn((batch * stride,), generator=g, device=dev) * 0.05
+    shape = (N, K) if layout == "nt" else (K, N)
+    B = flat.as_strided((batch, *shape), (stride, shape[1], 1))
+    C0 = torch.randn((batch, M, N), generator=g, device=dev)
+    bias = torch.randn((N,), generator=g, device=dev)
+    c = C0.clone()
+    print("split cut", M, N, K, batch, layout, gap, flush=True)
+    G.gemm(A, B, c, transB=layout == "nt", batch=batch, strideA=M * K, strideB=stride, strideC=M * N, alpha=0.5,
+           beta=0.5 if form.startswith("k") else 0.0, bias=bias, act=G.ACT_RELU)
+    for i in range(batch):
+        b = B[i].double().t().contiguous() if layout == "nt" else B[i].double()
+        ref = 0.5 * (A[i].double() @ b) + bias.double()
+        if form.startswith("k"):
+            ref += 0.5 * C0[i].double()
+        assert _rel(c[i], ref.clamp_min(0.0)) <= 1e-6  # 5e-7 of the product; the epilogue rounds twice more
+
+
 def test_split_parts_of_k_beyond_the_kept_scratch(dev):
     """Operands whose packed form exceeds the scratch a stream keeps (512 MiB) run in parts of K,
     each adding to C: beta once, bias and activation once, at the end."""

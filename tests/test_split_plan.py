@@ -1,0 +1,37 @@
+"""How fp32 products are cut for the bf16 matrix cores, on the CPU through the built library
+(tests/split_plan/split_plan.cpp): what the kernels assume of alignments, beta, slices and workspace
+holds for every part of every cut."""
+import os
+import re
+import subprocess
+
+import pytest
+
+from test_gemm_split_gpu import CUTS
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+DIR = os.path.join(ROOT, "tests", "split_plan")
+
+
+@pytest.fixture(scope="module")
+def plan():
+    subprocess.run(["make", "-s", "-C", DIR], check=True, capture_output=True)
+    return os.path.join(DIR, "_build", "split_plan")
+
+
+def test_every_part_of_every_cut_keeps_the_kernels_assumptions(plan):
+    r = subprocess.run([plan], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stdout[-4000:]
+    assert r.stdout.strip().endswith("0 violations")
+    seen = {k: int(v) for k, v in re.findall(r"(\w+) (\d+)", r.stdout.splitlines()[0])}
+    assert all(v > 500 for v in seen.values()), seen  # every form of cut was walked
+
+
+@pytest.mark.parametrize("M,N,K,batch,layout,gap,form", CUTS)
+def test_gpu_cases_reach_the_cuts_they_name(plan, M, N, K, batch, layout, gap, form):
+    out = subprocess.run([plan, *map(str, (M, N, K, batch, layout, gap))], capture_output=True, text=True).stdout
+    m = re.match(r"nb (\d+) kc (\d+) raw (\d) S (\d+)", out)
+    assert m, out
+    nb, kc, raw, S = map(int, m.groups())
+    assert {"batch": 1 < nb < batch, "single": nb == 1 < batch, "k": kc < K}[form.split("-")[0]]
+    assert raw == form.endswith("raw")
