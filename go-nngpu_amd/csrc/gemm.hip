@@ -1776,8 +1776,8 @@ template <bool VST, int ACT>
 __global__ void __launch_bounds__(256)
     splitk_reduce_kernel(const float *__restrict__ P, int S, long PS, long M, long N, float *C, long ldc,
                          float alpha, float beta, const float *__restrict__ bias, int act_rt, float act_alpha,
-                         const unsigned long long *gate, unsigned long long gate_seq) {
-  if (gate && *gate == gate_seq) return;  // the partials were not written (GemmParams)
+                         const SplitGate *gate, unsigned long long gate_seq) {
+  if (gate && split_fp32_needed(*gate, gate_seq)) return;  // the partials do not count
   const long MN = M * N;
   const int act = ACT == kActRuntime ? act_rt : ACT;
   const long step = (long)gridDim.x * blockDim.x;
@@ -1968,7 +1968,7 @@ bool takes_rows(const GemmDesc &d, const RowsPlan &rows, bool a_ok, bool b_ok, b
 // nothing.
 hipError_t run_split(const GemmDesc &d, const SplitCut &cut, bool vec, char *ws, hipStream_t s) {
   static std::atomic<unsigned long long> calls{0};
-  auto *gate = reinterpret_cast<unsigned long long *>(ws);
+  auto *gate = reinterpret_cast<SplitGate *>(ws);
   float *part = reinterpret_cast<float *>(ws + 256);
   char *packed = ws + 256 + (cut.plan.part_bytes + 255) / 256 * 256;
   for (long z = 0; z < d.batch; z += cut.nb)
@@ -1983,7 +1983,7 @@ hipError_t run_split(const GemmDesc &d, const SplitCut &cut, bool vec, char *ws,
       if (k + cut.kc < d.K) q.bias = nullptr, q.act = -1;
       SplitPlan plan = cut.plan;
       plan.S = split_slices(plan, q.K);
-      // a value no earlier call left in *gate; a chance match in fresh scratch only costs time
+      // a value no earlier call left in the gate; a chance match in fresh scratch only costs time
       const unsigned long long seq = ++calls;
       if (hipError_t e = launch_split(q, plan, packed, part, gate, seq, s)) return e;
       GemmParams p{};

@@ -3,6 +3,7 @@
 #pragma once
 
 #include "common.h"
+#include "split_gate.h"
 
 namespace gn {
 
@@ -46,10 +47,10 @@ bool cut_split(const GemmDesc &d, bool a_ok, bool b_ok, SplitCut *cut);
 inline long splitk_stride(long M, long N) { return (M * N + 3) / 4 * 4; }
 
 // Packs the operands into ws (plan.pack_bytes) and multiplies them into C (d.C with the
-// epilogue when plan.S == 1, else the partial products of the S slices into part). *gate
-// becomes seq when an operand holds a value the parts do not. Then d.C still holds what it held,
-// except with a raw B and S == 1 (which plan_split gives for beta == 0 only).
-hipError_t launch_split(const GemmDesc &d, const SplitPlan &plan, char *ws, float *part, unsigned long long *gate,
+// epilogue when plan.S == 1, else the partial products of the S slices into part). A word
+// of *gate becomes seq when an operand holds a value the parts do not. Then d.C still holds what it
+// held, except with a raw B and S == 1 (which plan_split gives for beta == 0 only).
+hipError_t launch_split(const GemmDesc &d, const SplitPlan &plan, char *ws, float *part, SplitGate *gate,
                         unsigned long long seq, hipStream_t s);
 
 }  // namespace gn

@@ -13,8 +13,8 @@
 //
 // Range: the packed parts are of x 2^16, so that the low parts of subnormals are whole bf16
 // subnormals, and a product takes this way only when every |x| < 2^36 (for K up to 2^20 no sum of
-// x 2^16 y 2^16 overflows). The pack kernel looks; otherwise, infinities and NaN included, the
-// product kernel returns and the fp32 kernels enqueued behind it run (GemmParams::gate).
+// x 2^16 y 2^16 overflows). The pack kernel looks, and the product kernel in a B that it splits itself;
+// otherwise, infinities and NaN included, the fp32 kernels enqueued behind them compute C (split_gate.h).
 //
 // Time, 4096^3 NN: pack 62-75 us (335 MB at copy rate), product 508 us = 270 TFLOP/s, 1.62 PFLOP/s of
 // bf16 products, which is the rate the board's power limit leaves the matrix cores; 928 -> 606 us
@@ -79,7 +79,7 @@ __device__ __forceinline__ Parts split8(const float (&x)[8], bool &bad) {
 // One K-tile of 64 rows per workgroup: with two or four K-tiles a workgroup the large operands
 // took as long, and the small ones longer (1024 x 1024: 13 against 9 us), for want of waves.
 __global__ void __launch_bounds__(256) split_pack_kernel(PackSide a, PackSide b, long K, int nkt, int ya,
-                                                         unsigned long long *flag, unsigned long long seq) {
+                                                         SplitGate *gate, unsigned long long seq) {
   const bool is_b = (int)blockIdx.y >= ya;
   const PackSide s = is_b ? b : a;
   const long y = is_b ? blockIdx.y - ya : blockIdx.y;
@@ -114,7 +114,7 @@ __global__ void __launch_bounds__(256) split_pack_kernel(PackSide a, PackSide b,
   char *d = s.dst + (long)blockIdx.z * s.dstride + (rb * nkt + blockIdx.x) * kSplitBlock + (g * 16 + (r & 15)) * 16;
 #pragma unroll
   for (int q = 0; q < 3; ++q) *reinterpret_cast<bf16x8_t *>(d + q * 1024) = o.p[q];
-  if (bad) *flag = seq;
+  if (bad) __hip_atomic_store(&gate->packed, seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // 16 bytes per lane from the buffer at voff + soff into LDS at lds + 16 * lane. Every offset is
@@ -157,7 +157,7 @@ gemm_split_kernel(GemmParams p, SplitArgs q) {
   static_assert((CA % NW == 0 || CA < 2 * NW) && CB % NW == 0, "tile shape");
   static_assert(WM * 16 * (BN + 4) * 4 <= NS * SLOT, "epilogue staging exceeds the ring");
   __shared__ __attribute__((aligned(1024))) char smem[NS * SLOT];
-  if (*p.gate == p.gate_seq) return;  // uniform: a value the split does not hold; the fp32 kernels run instead
+  if (split_product_skipped(*p.gate, p.gate_seq)) return;  // uniform: no workgroup of this launch writes that word
   int tm, tn;
   tile_coords(p, tm, tn);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -342,7 +342,7 @@ gemm_split_kernel(GemmParams p, SplitArgs q) {
     for (int t = 0; t < nt; ++t) step(t, 0);
   }
   __syncthreads();
-  if (BSRC && bad) *const_cast<unsigned long long *>(p.gate) = p.gate_seq;
+  if (BSRC && bad) __hip_atomic_store(&p.gate->multiplied, p.gate_seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
@@ -421,7 +421,7 @@ bool plan_split(const GemmDesc &d, long nb, long kc, SplitPlan *out) {
   return true;
 }
 
-hipError_t launch_split(const GemmDesc &d, const SplitPlan &plan, char *ws, float *part, unsigned long long *gate,
+hipError_t launch_split(const GemmDesc &d, const SplitPlan &plan, char *ws, float *part, SplitGate *gate,
                         unsigned long long seq, hipStream_t s) {
   SplitArgs q{};
   q.nkt = (int)((d.K + 31) / 32);

@@ -5,6 +5,7 @@
 #include "act.h"
 #include "common.h"
 #include "ring_plan.h"
+#include "split_gate.h"
 
 namespace gn {
 namespace {
@@ -31,15 +32,14 @@ struct GemmParams {
   int tiles_m, tiles_n;
   int group_m;  // tile rows per raster group (tile_coords); 0 selects the default of 4
   // An fp32 product on the bf16 matrix cores (gemm_split.hip) and its fp32 kernels are both
-  // enqueued; *gate == gate_seq says that an operand holds a value the split does not. The
-  // split kernels then write nothing and the fp32 kernels (GATED) run, else the other way
-  // round.
-  const unsigned long long *gate;
+  // enqueued; the gate says whose result counts (split_gate.h). The fp32 kernels (GATED) return at
+  // once where the split's does.
+  SplitGate *gate;
   unsigned long long gate_seq;
 };
 
 // False in an fp32 kernel that stands behind a split product whose operands allowed it.
-__device__ __forceinline__ bool fp32_needed(const GemmParams &p) { return *p.gate == p.gate_seq; }
+__device__ __forceinline__ bool fp32_needed(const GemmParams &p) { return split_fp32_needed(*p.gate, p.gate_seq); }
 
 // ------------------------------------------------------------------ epilogue
 // Workgroup barrier that orders LDS accesses only (s_waitcnt lgkmcnt(0); s_barrier).

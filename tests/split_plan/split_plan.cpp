@@ -8,6 +8,9 @@
 //  * B split by the product kernel without slices of K (C is written before the values are known):
 //    the part's beta is 0;
 //  * no slice is empty, and the workspace holds the part's packed operands and partial products.
+// And of the gate (split_gate.h): nothing that workgroups of the product kernel write changes what
+// others of the same launch read, and whichever kernel finds a value stops the reduce and calls for the
+// fp32 kernels, for this call only.
 // Exit 0: no violation; 1: violations. Prints how many cuts of each form it saw. With arguments M N K
 // batch layout gap (nn, nt, tn or tt; gap: elements between the batches' B) it prints that product's cut.
 #include <cstdio>
@@ -91,6 +94,13 @@ GemmDesc product(long M, long N, long K, long batch, bool ta, bool tb, long gap)
 }
 
 }  // namespace
+
+constexpr unsigned long long kSeq = 7, kOld = 6;
+// The product kernel's test reads the same before and after workgroups of the same launch wrote.
+static_assert(!split_product_skipped({kOld, kOld}, kSeq) && !split_product_skipped({kOld, kSeq}, kSeq), "uniform");
+static_assert(split_product_skipped({kSeq, kOld}, kSeq) && split_product_skipped({kSeq, kSeq}, kSeq), "uniform");
+static_assert(split_fp32_needed({kSeq, kOld}, kSeq) && split_fp32_needed({kOld, kSeq}, kSeq), "either finder");
+static_assert(!split_fp32_needed({kOld, kOld}, kSeq), "an earlier call's values");
 
 int main(int argc, char **argv) {
   if (argc == 7) {

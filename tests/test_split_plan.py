@@ -27,6 +27,16 @@ def test_every_part_of_every_cut_keeps_the_kernels_assumptions(plan):
     assert all(v > 500 for v in seen.values()), seen  # every form of cut was walked
 
 
+def test_each_gate_word_is_written_by_one_kernel_and_tested_by_later_ones():
+    src = open(os.path.join(ROOT, "go-nngpu_amd", "csrc", "gemm_split.hip")).read()
+    pack, product = src.split("split_pack_kernel(", 1)[1].split("gemm_split_kernel(", 1)
+    product = product.split("hipError_t launch_tile", 1)[0]
+    assert re.findall(r"gate->(\w+)", pack) == ["packed"]
+    # the product kernel writes the one word and tests the gate through the function above only
+    assert re.findall(r"gate->(\w+)", product) == ["multiplied"]
+    assert re.findall(r"\w+\(\*p\.gate|\*p\.gate", product) == ["split_product_skipped(*p.gate"]
+
+
 @pytest.mark.parametrize("M,N,K,batch,layout,gap,form", CUTS)
 def test_gpu_cases_reach_the_cuts_they_name(plan, M, N, K, batch, layout, gap, form):
     out = subprocess.run([plan, *map(str, (M, N, K, batch, layout, gap))], capture_output=True, text=True).stdout
