@@ -233,10 +233,14 @@ __global__ void __launch_bounds__(WM * WN * 64) gemm_f16_kernel(GemmParams p) {
 //    16-byte fragment reads (25 M conflict cycles per operand at 4096^3), so both tiles
 //    are stored transposed (four 4-byte writes, conflict-free for these loaders) and read
 //    as M/N-contiguous ones: 4096^3 NT 1045 -> 1020 us; NN, TN and TT do not gain.
-// GATED: stands behind a split product (GemmParams::gate); a template argument because the
-// gate's load, ahead of the other arguments', cost the 12 us batched products half a microsecond.
-template <int BM, int BN, int BK, int WM, int WN, bool TA, bool TB, bool VEC, bool GATED>
-__global__ void __launch_bounds__(WM * WN * 64) gemm_f32_kernel(GemmParams p) {
+// One tile: w is its linear id, z its batch.
+template <int BM, int BN, int BK, int WM, int WN, bool TA, bool TB>
+constexpr int f32_staged_floats() {
+  constexpr bool XT = !TA && TB && BK == 16, MA = TA || XT, MB = !TB || XT;
+  return 2 * ((MA ? BK * (BM + 4) : BM * (BK + 4)) + (MB ? BK * (BN + 4) : BN * (BK + 4)));
+}
+template <int BM, int BN, int BK, int WM, int WN, bool TA, bool TB, bool VEC>
+__device__ __forceinline__ void f32_staged_tile(const GemmParams &p, int w, long z, float *smem) {
   constexpr int NT = WM * WN * 64;
   constexpr int WTM = BM / WM, WTN = BN / WN;
   constexpr int FM = WTM / 16, FN = WTN / 16;
@@ -247,13 +251,11 @@ __global__ void __launch_bounds__(WM * WN * 64) gemm_f32_kernel(GemmParams p) {
   constexpr int PB = MB ? BN + 4 : BK + 4;
   constexpr int A_ELEMS = MA ? BK * PA : BM * PA;
   constexpr int B_ELEMS = MB ? BK * PB : BN * PB;
-  __shared__ __attribute__((aligned(16))) float smem[2 * (A_ELEMS + B_ELEMS)];
-  if (GATED && !fp32_needed(p)) return;
+  static_assert(2 * (A_ELEMS + B_ELEMS) == f32_staged_floats<BM, BN, BK, WM, WN, TA, TB>(), "LDS size");
 
   int tm, tn;
-  tile_coords(p, tm, tn);
+  tile_coords(p, w, tm, tn);
   const long m0 = (long)tm * BM, n0 = (long)tn * BN;
-  const long z = blockIdx.z;
   const float *A = static_cast<const float *>(p.A) + z * p.strideA;
   const float *B = static_cast<const float *>(p.B) + z * p.strideB;
 
@@ -338,6 +340,18 @@ __global__ void __launch_bounds__(WM * WN * 64) gemm_f32_kernel(GemmParams p) {
 
   static_assert(WM * 16 * (BN + 4) <= 2 * (A_ELEMS + B_ELEMS), "epilogue staging exceeds LDS");
   store_tile_rows<BM, BN, WM, WN>(p, m0, n0, z, smem, acc);
+}
+
+// GATED: stands behind a split product (GemmParams::gate); a template argument because the
+// gate's load, ahead of the other arguments', cost the 12 us batched products half a microsecond.
+template <int BM, int BN, int BK, int WM, int WN, bool TA, bool TB, bool VEC, bool GATED>
+__global__ void __launch_bounds__(WM * WN * 64) gemm_f32_kernel(GemmParams p) {
+  __shared__ __attribute__((aligned(16))) float smem[f32_staged_floats<BM, BN, BK, WM, WN, TA, TB>()];
+  auto tile = [&](const GemmParams &q, int w, long z) {
+    f32_staged_tile<BM, BN, BK, WM, WN, TA, TB, VEC>(q, w, z, smem);
+  };
+  if constexpr (GATED) gated_tiles<TA, TB>(p, tile);
+  else tile(p, blockIdx.x, blockIdx.z);
 }
 
 // The small-product kernels' end: wave w's partial tile goes to red[w], the workgroup adds
@@ -1244,18 +1258,21 @@ gemm_f32_ring_kernel(GemmParams p) {
   constexpr int FM = BM / WM / 16, FN = BN / WN / 16;
   constexpr int RING = NS * 2 * (BM + BN) * 16 * 4;  // NS slots of two K-tiles of A and B
   __shared__ __attribute__((aligned(1024))) char smem[RING];
-  if (GATED && !fp32_needed(p)) return;
-  int tm, tn;
-  tile_coords(p, tm, tn);
-  float4_t acc[FM][FN];
+  auto tile = [&](const GemmParams &q, int w, long z) {
+    int tm, tn;
+    tile_coords(q, w, tm, tn);
+    float4_t acc[FM][FN];
 #pragma unroll
-  for (int i = 0; i < FM; ++i)
+    for (int i = 0; i < FM; ++i)
 #pragma unroll
-    for (int j = 0; j < FN; ++j) acc[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
-  const long m0 = (long)tm * BM, n0 = (long)tn * BN, z = blockIdx.z;
-  ring_mainloop_f32<BM, BN, WM, WN, TA, TB, NS>(p, m0, n0, z, (int)((p.K + 15) / 16), smem, acc);
-  static_assert(WM * 16 * (BN + 4) * 4 <= RING, "epilogue staging exceeds the ring");
-  store_tile_rows<BM, BN, WM, WN>(p, m0, n0, z, reinterpret_cast<float *>(smem), acc);
+      for (int j = 0; j < FN; ++j) acc[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
+    const long m0 = (long)tm * BM, n0 = (long)tn * BN;
+    ring_mainloop_f32<BM, BN, WM, WN, TA, TB, NS>(q, m0, n0, z, (int)((q.K + 15) / 16), smem, acc);
+    static_assert(WM * 16 * (BN + 4) * 4 <= RING, "epilogue staging exceeds the ring");
+    store_tile_rows<BM, BN, WM, WN>(q, m0, n0, z, reinterpret_cast<float *>(smem), acc);
+  };
+  if constexpr (GATED) gated_tiles<TA, TB>(p, tile);
+  else tile(p, blockIdx.x, blockIdx.z);
 }
 
 // ------------------------------------------------------------------ dispatch
@@ -1293,11 +1310,18 @@ hipError_t launch_small_code(int code, const GemmParams &p, long batch, hipStrea
   }
 }
 
+template <bool GATED>
+dim3 f32_grid(const GemmParams &p, long batch) {
+  const long tiles = (long)p.tiles_m * p.tiles_n;
+  if (GATED) return dim3((unsigned)std::min<long>(tiles * p.nz, kGatedGrid));
+  return dim3((unsigned)tiles, 1, (unsigned)batch);
+}
+
 template <int BM, int BN, int BK, int WM, int WN, bool TA, bool TB, bool VEC, bool GATED = false>
 hipError_t launch_f32(GemmParams p, long batch, hipStream_t s) {
   p.tiles_m = (int)((p.M + BM - 1) / BM);
   p.tiles_n = (int)((p.N + BN - 1) / BN);
-  dim3 grid((unsigned)(p.tiles_m * p.tiles_n), 1, (unsigned)batch);
+  const dim3 grid = f32_grid<GATED>(p, batch);
   hipLaunchKernelGGL((gemm_f32_kernel<BM, BN, BK, WM, WN, TA, TB, VEC, GATED>), grid, dim3(WM * WN * 64), 0, s, p);
   return hipGetLastError();
 }
@@ -1315,7 +1339,7 @@ template <int BM, int BN, int WM, int WN, bool TA, bool TB, int WPE = 2, int NS 
 hipError_t launch_f32_ring(GemmParams p, long batch, hipStream_t s) {
   p.tiles_m = (int)((p.M + BM - 1) / BM);
   p.tiles_n = (int)((p.N + BN - 1) / BN);
-  dim3 grid((unsigned)(p.tiles_m * p.tiles_n), 1, (unsigned)batch);
+  const dim3 grid = f32_grid<GATED>(p, batch);
   hipLaunchKernelGGL((gemm_f32_ring_kernel<BM, BN, WM, WN, TA, TB, WPE, NS, GATED>), grid, dim3(WM * WN * 64), 0, s, p);
   return hipGetLastError();
 }
@@ -1775,9 +1799,7 @@ __global__ void gemm_k0_kernel(GemmParams p, long batch) {
 template <bool VST, int ACT>
 __global__ void __launch_bounds__(256)
     splitk_reduce_kernel(const float *__restrict__ P, int S, long PS, long M, long N, float *C, long ldc,
-                         float alpha, float beta, const float *__restrict__ bias, int act_rt, float act_alpha,
-                         const SplitGate *gate, unsigned long long gate_seq) {
-  if (gate && split_fp32_needed(*gate, gate_seq)) return;  // the partials do not count
+                         float alpha, float beta, const float *__restrict__ bias, int act_rt, float act_alpha) {
   const long MN = M * N;
   const int act = ACT == kActRuntime ? act_rt : ACT;
   const long step = (long)gridDim.x * blockDim.x;
@@ -1832,7 +1854,7 @@ hipError_t launch_splitk_reduce(const float *P, int S, const GemmParams &p, hipS
   const long PS = splitk_stride(p.M, p.N);
   auto go = [&](auto v, auto a) {
     hipLaunchKernelGGL((splitk_reduce_kernel<decltype(v)::value, decltype(a)::value>), grid, block, 0, s, P, S, PS,
-                       p.M, p.N, p.C, p.ldc, p.alpha, p.beta, p.bias, p.act, p.act_alpha, p.gate, p.gate_seq);
+                       p.M, p.N, p.C, p.ldc, p.alpha, p.beta, p.bias, p.act, p.act_alpha);
   };
   auto pick = [&](auto v) {
     switch (p.act) {
@@ -1913,29 +1935,41 @@ double f32_cores_us(const GemmDesc &d, bool a_ok, bool b_ok) {
   return us;
 }
 
-// The fp32 kernels behind a split product (GemmParams::gate): 128 x 128 ring tiles and the last
-// K % 32 on the register-staged kernel, or that kernel alone where the ring does not go.
+// The fp32 kernels behind a split product (GemmParams::gate), in the split's slices of K: the ring on
+// the better of two tiles with the last K % 32 of an unsliced product on the register-staged kernel,
+// or that kernel alone where the ring does not go. With a value the split does not hold a call
+// then takes (us, against the fp32 path alone; always 128 x 128 tiles in one launch in brackets) 4096^3
+// 994 / 927, 512 x 4096 x 11008 368 / 350 [666], 1100 x 1100 x 4000 116 / 127 [259], 200 x 1000 x 2000 30 / 42
+// [138]; where the value is in a raw B the split's product is made first: 512 x 11008 x 4096 618 / 367 [690].
+// Unaligned operands are read element by element (packing them would be one more launch for every
+// product): 777 x 1234 x 4099 195 / 110 [310] and up to twice the fp32 path.
 template <bool TA, bool TB, bool VEC>
 hipError_t launch_f32_behind(const GemmParams &p, long batch, hipStream_t s) {
+  const long nz = batch * p.slices;
+  const F32Costs cost = f32_ring_costs(p.M, p.N, nz);
+  const bool wide = cost.c128 <= cost.c64;
   if constexpr (VEC) {
-    if (ring_offsets_fit(p) && p.K >= 32) {
-      const long kt = p.K % 32;
+    const long kt = p.K % 32;
+    if (ring_offsets_fit(p) && p.K >= 32 && (kt == 0 || p.slices == 1)) {
       GemmParams head = p, tail = p;
       head.K = p.K - kt;
       if (kt) {
         head.bias = nullptr;
         head.act = -1;
       }
-      if (hipError_t e = launch_f32_ring<128, 128, 2, 2, TA, TB, 2, 2, true>(head, batch, s)) return e;
+      if (hipError_t e = wide ? launch_f32_ring<128, 128, 2, 2, TA, TB, 2, 2, true>(head, nz, s)
+                              : launch_f32_ring<64, 64, 2, 2, TA, TB, 2, 2, true>(head, nz, s))
+        return e;
       if (!kt) return hipSuccess;
       tail.K = kt;
       tail.beta = 1.0f;
       tail.A = static_cast<const float *>(p.A) + (TA ? head.K * p.lda : head.K);
       tail.B = static_cast<const float *>(p.B) + (TB ? head.K : head.K * p.ldb);
-      return launch_f32<64, 64, 16, 2, 2, TA, TB, true, true>(tail, batch, s);
+      return launch_f32<64, 64, 16, 2, 2, TA, TB, true, true>(tail, nz, s);
     }
   }
-  return launch_f32<64, 64, 16, 2, 2, TA, TB, VEC, true>(p, batch, s);
+  return wide ? launch_f32<128, 128, 16, 2, 2, TA, TB, VEC, true>(p, nz, s)
+              : launch_f32<64, 64, 16, 2, 2, TA, TB, VEC, true>(p, nz, s);
 }
 
 template <bool VEC>
@@ -1962,10 +1996,10 @@ bool takes_rows(const GemmDesc &d, const RowsPlan &rows, bool a_ok, bool b_ok, b
   return d.M <= 32 || rows.us < 1.15 * (f32_cores_us(d, a_ok, b_ok) + 3.0);
 }
 
-// Enqueues the product by `cut` with ws (cut.ws_bytes) as its workspace. Behind every part the
-// fp32 kernels are enqueued too; they return at once unless an operand holds a value the split
-// does not (an infinity, a NaN, or 2^36 and more), in which case the part's split kernels wrote
-// nothing.
+// Enqueues the product by `cut` with ws (cut.ws_bytes) as its workspace. Behind every part's split
+// kernels the fp32 kernels are enqueued too; they return at once unless an operand holds a value the
+// split does not (an infinity, a NaN, or 2^36 and more), in which case they compute C, or the partial
+// products that the reduce adds.
 hipError_t run_split(const GemmDesc &d, const SplitCut &cut, bool vec, char *ws, hipStream_t s) {
   static std::atomic<unsigned long long> calls{0};
   auto *gate = reinterpret_cast<SplitGate *>(ws);
@@ -1994,9 +2028,21 @@ hipError_t run_split(const GemmDesc &d, const SplitCut &cut, bool vec, char *ws,
       p.alpha = q.alpha; p.beta = q.beta; p.act = q.act; p.act_alpha = q.act_alpha;
       p.gate = gate;
       p.gate_seq = seq;
+      p.slices = plan.S;
+      p.nz = (int)(q.batch * plan.S);
+      GemmParams r = p;
+      if (plan.S > 1) {
+        r.C = part;
+        r.ldc = q.N;
+        r.strideC = splitk_stride(q.M, q.N);
+        r.alpha = 1.0f;
+        r.beta = 0.0f;
+        r.bias = nullptr;
+        r.act = -1;
+      }
+      if (hipError_t e = vec ? dispatch_behind<true>(q.ta, q.tb, r, q.batch, s) : dispatch_behind<false>(q.ta, q.tb, r, q.batch, s)) return e;
       if (plan.S > 1)
         if (hipError_t e = launch_splitk_reduce(part, plan.S, p, s)) return e;
-      if (hipError_t e = vec ? dispatch_behind<true>(q.ta, q.tb, p, q.batch, s) : dispatch_behind<false>(q.ta, q.tb, p, q.batch, s)) return e;
     }
   return hipSuccess;
 }

@@ -18,6 +18,7 @@ typedef __fp16 trh4_t __attribute__((__vector_size__(4 * sizeof(__fp16))));
 typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
 
 #define LDS_AS __attribute__((address_space(3)))
+#define CONST_AS __attribute__((address_space(4)))
 
 struct GemmParams {
   const void *A;
@@ -36,10 +37,24 @@ struct GemmParams {
   // once where the split's does.
   SplitGate *gate;
   unsigned long long gate_seq;
+  int slices, nz;  // GATED: slices of K per batch; batch x slices
 };
 
 // False in an fp32 kernel that stands behind a split product whose operands allowed it.
 __device__ __forceinline__ bool fp32_needed(const GemmParams &p) { return split_fp32_needed(*p.gate, p.gate_seq); }
+
+// p for slice z % slices of K of batch z / slices, cut as the split product's slices are (whole 32-k
+// tiles), so that its partial products take the places of the split's.
+template <bool TA, bool TB>
+__device__ __forceinline__ GemmParams slice_of(GemmParams p, int z) {
+  const int S = p.slices, zb = z / S, sl = z - zb * S, nkt = (int)((p.K + 31) / 32);
+  const long k0 = (long)sl * nkt / S * 32, k1 = min((long)(sl + 1) * nkt / S * 32, p.K);
+  p.A = static_cast<const float *>(p.A) + zb * p.strideA + (TA ? k0 * p.lda : k0);
+  p.B = static_cast<const float *>(p.B) + zb * p.strideB + (TB ? k0 : k0 * p.ldb);
+  p.strideA = p.strideB = 0;
+  p.K = k1 - k0;
+  return p;
+}
 
 // ------------------------------------------------------------------ epilogue
 // Workgroup barrier that orders LDS accesses only (s_waitcnt lgkmcnt(0); s_barrier).
@@ -156,12 +171,11 @@ __device__ __forceinline__ void store_tile_rows(const GemmParams &p, long m0, lo
   });
 }
 
-// Grouped + XCD-aware mapping of the linear workgroup id to a (tile_m, tile_n) pair.
-__device__ __forceinline__ void tile_coords(const GemmParams &p, int &tm, int &tn) {
+// Grouped + XCD-aware mapping of the linear workgroup id w to a (tile_m, tile_n) pair.
+__device__ __forceinline__ void tile_coords(const GemmParams &p, int w, int &tm, int &tn) {
   // Workgroup w runs on XCD w % 8; give XCD x the contiguous tile range
   // [x*base + min(x, rem), ...) of base (+1 for the first rem XCDs) tiles.
   const int total = p.tiles_m * p.tiles_n;
-  int w = blockIdx.x;
   {
     const int base = total >> 3, rem = total & 7, x = w & 7;
     w = x * base + min(x, rem) + (w >> 3);
@@ -174,6 +188,27 @@ __device__ __forceinline__ void tile_coords(const GemmParams &p, int &tm, int &t
   const int r = w - group * in_group;
   tm = first_m + r % gsize;
   tn = r / gsize;
+}
+__device__ __forceinline__ void tile_coords(const GemmParams &p, int &tm, int &tn) { tile_coords(p, blockIdx.x, tm, tn); }
+
+// A GATED kernel's tiles, body(p of the slice, tile, z) for each: its workgroups, at most
+// kGatedGrid, take them in turn. An empty workgroup costs about a nanosecond of a product whose
+// split counts (512 x 4096 x 11008: 2048 of them 4 us).
+constexpr int kGatedGrid = 512;
+template <bool TA, bool TB, typename Body>
+__device__ __forceinline__ void gated_tiles(const GemmParams &p, Body &&body) {
+  if (!fp32_needed(p)) return;
+  // The kernel's arguments (p is the only one), read again for every tile: kept beside a tile's own
+  // they take more scalar registers than there are.
+  auto *args = (const CONST_AS GemmParams *)__builtin_amdgcn_kernarg_segment_ptr();
+  for (long u = blockIdx.x;; u += gridDim.x) {
+    asm volatile("" : "+s"(args));
+    const GemmParams q = *(const GemmParams *)args;
+    const int tiles = q.tiles_m * q.tiles_n, z = (int)(u / tiles);
+    if (z >= q.nz) return;
+    body(slice_of<TA, TB>(q, z), (int)(u - (long)z * tiles), z);
+    __syncthreads();  // before the next tile's copies into LDS
+  }
 }
 
 typedef int i32x4_t __attribute__((ext_vector_type(4)));

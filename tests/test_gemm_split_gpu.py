@@ -199,6 +199,65 @@ def test_split_values_it_does_not_hold(dev, M, N, K, value, side, beta):
     assert _rel(c, A.double() @ B.double()) <= 5e-7
 
 
+@pytest.mark.parametrize("tA,tB", VARIANTS)
+@pytest.mark.parametrize("M,N,K", [(1100, 1100, 4000), (1100, 1100, 4004), (2048, 2048, 1044), (4100, 4100, 1024), (200, 1000, 2000),
+                                   (1023, 1025, 4001), (3001, 2999, 517)])
+def test_split_values_it_does_not_hold_on_every_fp32_form(dev, M, N, K, tA, tB):
+    """The fp32 kernels behind a split product in its slices of K and in one launch, on both tiles,
+    with a remainder of K % 32, aligned or not: alpha, beta, bias and activation once."""
+    import torch
+
+    g = torch.Generator(device=dev).manual_seed(M + K)
+    A = torch.randn((M, K), generator=g, device=dev)
+    B = torch.randn((K, N), generator=g, device=dev)
+    A[3, K - 1] = float("inf")
+    B[K - 1, 5] = float("nan")
+    B[1, 7] = 2.0**37
+    C0 = torch.randn((M, N), generator=g, device=dev)
+    bias = torch.randn((N,), generator=g, device=dev)
+    c = C0.clone()
+    print("split fp32 form", M, N, K, tA, tB, flush=True)
+    G.gemm(_stored(A, tA), _stored(B, tB), c, transA=tA, transB=tB, alpha=0.5, beta=2.0, bias=bias, act=G.ACT_RELU)
+    ref = 0.5 * (A.double() @ B.double()) + 2.0 * C0.double() + bias.double()
+    # the library's ReLU is fmaxf(x, 0): 0 for NaN
+    ref = torch.where(torch.isnan(ref), torch.zeros_like(ref), ref.clamp_min(0.0))
+    fine = torch.isfinite(ref)
+    assert torch.equal(torch.isinf(c), torch.isinf(ref)) and not torch.isnan(c).any()
+    col = torch.ones(N, dtype=torch.bool, device=dev)
+    col[7] = False  # 2^37 times a normal value: its column apart
+    for part in (fine & col, fine & ~col):
+        assert _rel(c[part], ref[part]) <= 2e-6
+
+
+@pytest.mark.parametrize("M,N,K", [(256, 4096, 4096), (200, 1000, 2000), (1100, 1100, 4000)])
+def test_split_values_it_does_not_hold_cost_a_second_product_at_most(dev, M, N, K):
+    """Few tiles and a long K: the fp32 kernels behind the split run in its slices of K, as the ordinary
+    path would. (In one launch they took these calls from 42-128 us to 138-300, 3.6 to 4.9 times the same
+    call with finite operands; now 1.1 to 2.3 times.)"""
+    import torch
+
+    g = torch.Generator(device=dev).manual_seed(M)
+    A = torch.randn((M, K), generator=g, device=dev)
+    B = torch.randn((K, N), generator=g, device=dev)
+    c = torch.empty((M, N), device=dev)
+    times = {}
+    for kind in ("finite", "infinite"):
+        if kind == "infinite":
+            B[1, 1] = float("inf")
+        start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        rounds = []
+        for _ in range(5):
+            torch.cuda._sleep(1000000)  # the calls queue up behind it
+            start.record()
+            for _ in range(10):
+                G.gemm(A, B, c)
+            end.record()
+            torch.cuda.synchronize()
+            rounds.append(start.elapsed_time(end))
+        times[kind] = sorted(rounds)[2]
+    assert times["infinite"] <= 3.0 * times["finite"], times
+
+
 @pytest.mark.parametrize("scale", [2.0**-140, 2.0**-100, 2.0**-60, 2.0**35])
 def test_split_range(dev, scale):
     """Rows of very small values (subnormal ones among them) and of the largest the split holds
