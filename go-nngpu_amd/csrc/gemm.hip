@@ -416,6 +416,11 @@ __device__ __forceinline__ void small_reduce_store(const GemmParams &p, float4_t
 // 1000 NN 5.9 -> 3.7. The KW partial tiles are added in LDS in wave order before
 // the epilogue (small_reduce_store), so each element's summation order depends on K and KW
 // alone: the same for all four transpose layouts, aligned or not.
+// An MFMA rounds its sum once per product, so a long sum costs precision: the steps of a batch go into
+// sums of their own (32 x 32 tiles, whose registers the third and fourth cost 10%: two), added at the end.
+// Relative error with one sum per wave -> now: fp32 512^3 2.1e-7 -> 1.5e-7, 100 x 130 x 1000 2.8e-7 ->
+// 1.5e-7, 255^2 x 2001 2.9e-7 -> 1.6e-7. At least two waves per SIMD, so that the compiler keeps the
+// sums in the MFMAs' own VGPRs: in AGPRs it copied them around every chain (5-10% of a call).
 // Per element type: the fragment vector V (E elements per lane and K step of KS elements)
 // and the MFMA steps MPS of one K step.
 template <typename T>
@@ -438,7 +443,8 @@ struct SmallOps<_Float16> {
 };
 
 template <typename T, int KW, int FM, int FN, bool TA, bool TB, bool VEC, int KB>
-__global__ void __launch_bounds__(KW * 64) gemm_small_kernel(GemmParams p) {
+__global__ void __launch_bounds__(KW * 64) __attribute__((amdgpu_waves_per_eu(KW > 8 ? KW / 4 : 2)))
+gemm_small_kernel(GemmParams p) {
   typedef SmallOps<T> Ops;
   typedef typename Ops::V V;
   constexpr int NF = FM * FN, U = KB / Ops::KS, E = Ops::E, KS = Ops::KS;  // KB elements of K per load batch
@@ -512,18 +518,21 @@ __global__ void __launch_bounds__(KW * 64) gemm_small_kernel(GemmParams p) {
     for (int j = 0; j < FN; ++j) be[j] = frag_end(B, p.ldb, TB, vb[j]);
   }
 
-  float4_t acc[FM][FN];
+  constexpr int NA = NF > 2 ? 2 : U;
+  float4_t acc[NA][FM][FN];  // a sum of its own for each step of a batch
 #pragma unroll
-  for (int i = 0; i < FM; ++i)
+  for (int u = 0; u < NA; ++u)
 #pragma unroll
-    for (int j = 0; j < FN; ++j) acc[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
-  auto multiply = [&](const V(&af)[FM], const V(&bf)[FN]) {
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j) acc[u][i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
+  auto multiply = [&](const V(&af)[FM], const V(&bf)[FN], float4_t(&c)[FM][FN]) {
 #pragma unroll
     for (int s = 0; s < Ops::MPS; ++s)
 #pragma unroll
       for (int i = 0; i < FM; ++i)
 #pragma unroll
-        for (int j = 0; j < FN; ++j) acc[i][j] = Ops::mma(af[i], bf[j], s, acc[i][j]);
+        for (int j = 0; j < FN; ++j) c[i][j] = Ops::mma(af[i], bf[j], s, c[i][j]);
   };
   auto batch = [&](int t0, auto part_c) {
     constexpr bool PART = decltype(part_c)::value;  // fewer than U steps are left: the rest count as zeros
@@ -550,14 +559,21 @@ __global__ void __launch_bounds__(KW * 64) gemm_small_kernel(GemmParams p) {
 #pragma unroll
           for (int e = 0; e < E; ++e) bf[u][j][e] = live ? bf[u][j][e] : T(0);
       }
-      multiply(af[u], bf[u]);
+      multiply(af[u], bf[u], acc[u % NA]);
+      __builtin_amdgcn_sched_barrier(0);  // in the order of the loads
     }
   };
   int t0 = sb;
   for (; t0 + U <= fe; t0 += U) batch(t0, std::false_type{});
   if (t0 < fe) batch(t0, std::true_type{});
-  if (se > fe) multiply(ae, be);
-  small_reduce_store<KW, FM, FN>(p, red, acc, m0, n0, z);
+  if (se > fe) multiply(ae, be, acc[NA - 1]);
+#pragma unroll
+  for (int u = 1; u < NA; ++u)
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j) acc[0][i][j] = acc[0][i][j] + acc[u][i][j];
+  small_reduce_store<KW, FM, FN>(p, red, acc[0], m0, n0, z);
 }
 
 // ------------------------------------------------------------------ fp16 DMA-ring kernel
@@ -1296,8 +1312,8 @@ hipError_t launch_small(GemmParams p, long batch, hipStream_t s) {
 
 // The small-product kernel of shape code 100 KW + 10 FM + FN; hipErrorInvalidValue for
 // another code. Load batches of 64 elements of K; 48 for fp32 on 32 x 16 tiles, whose waves
-// hold few K steps (256 x 512 x 784: 5.8 us against 6.3 with 64; 128 for 16 waves took 16 x 16 x 4096 from
-// 13.3 to 15.3).
+// hold few K steps (63 shapes, warm: 0.98 of the time with 64 in NN, 0.99 in the other layouts, and level
+// with operands from HBM; 128 for 16 waves took 16 x 16 x 4096 from 13.3 us to 15.3).
 template <typename T, bool TA, bool TB, bool VEC>
 hipError_t launch_small_code(int code, const GemmParams &p, long batch, hipStream_t s) {
   switch (code) {
@@ -1590,7 +1606,7 @@ hipError_t launch_f32_ring_best(const GemmParams &p, long batch, hipStream_t s) 
 // 32 ones leave the waves little to do (512^2 x 128: 4.1 against 4.5 us), 16 x 16 up to 2 steps.
 // Four waves split K; on 16 x 16 tiles 8 from 96 steps and 16 from 256 (up to 1024
 // waves in all): level there (256^2 x 2048: 7.5 / 7.9 / 8.6 us with 4 / 8 / 16; 64 x 128 x 1000: 4.4 /
-// 5.3 / 5.7) and their sums are shorter.
+// 5.3 / 5.7) and their sums are shorter (the sums of a wave: gemm_small_kernel).
 inline int f32_small_tile(long M, long N, long K, long batch, bool ta, bool tb) {
   if (const int c = skinny_tile(M, N, K, batch, false, ta, tb)) return c;
   const long tiles64 = ((M + 63) / 64) * ((N + 63) / 64) * batch;

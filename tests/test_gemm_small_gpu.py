@@ -43,3 +43,20 @@ def test_small_products(dev, shape, dtype, pad):
             a64, b64 = (a.t() if ta else a).cpu().double(), (b.t() if tb else b).cpu().double()
             bound = (k + 2) * 2.0**-24 * (a64.abs() @ b64.abs())
             assert bool(((c.cpu().double() - a64 @ b64).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("m,n,k", [(512, 512, 512), (384, 500, 700), (100, 130, 1000), (1, 1000, 1000), (64, 128, 784),
+                                   (255, 255, 2001), (256, 512, 784), (40, 1000, 600), (200, 24, 1250)])
+def test_small_products_sum_k_in_short_chains(dev, m, n, k):
+    """An fp32 MFMA rounds its sum once per product; a chain of c of them is off by about 2.5e-8
+    sqrt(c / 2) of the result for normal operands (the rms of a rounding, times the growth of the
+    partial sums). Chains of at most 64 products and the sum of the chains: 1.4e-7 to 1.6e-7; with
+    K split over four waves of one chain each these products were 2.0e-7 to 2.9e-7 off."""
+    import torch
+
+    g = torch.Generator(device=dev).manual_seed(k)
+    a, b = torch.randn((m, k), generator=g, device=dev), torch.randn((k, n), generator=g, device=dev)
+    c = torch.empty((m, n), device=dev)
+    G.gemm(a, b, c)
+    ref = a.double() @ b.double()
+    assert float((c.double() - ref).norm() / ref.norm()) <= 1.85e-7
