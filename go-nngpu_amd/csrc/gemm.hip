@@ -412,8 +412,10 @@ __device__ __forceinline__ void small_reduce_store(const GemmParams &p, float4_t
 // 10-20% slower: fewer waves fit). What bounds it is the latency of those load batches and the
 // instructions that address them, so whole K steps are loaded without bounds checks, from 32-bit
 // lane offsets that are computed once (rows past the product read its last one), and only a last,
-// partial step is masked: fp32 256 x 512 x 784 8.3 -> 5.8 us, 512^3 6.9 -> 5.8, fp16 100 x 136 x
-// 1000 NN 5.9 -> 3.7. The KW partial tiles are added in LDS in wave order before
+// partial step is masked; the whole steps after the last full batch have code for their exact number
+// (loading a full batch of which some count as zeros took a tenth of the shortest calls: 256 x 192 x 96
+// 3.6 us against 3.3): fp32 256 x 512 x 784 8.3 -> 5.7 us, 512^3 7.1 -> 6.3, fp16 100 x 136 x 1000 NN 5.9 ->
+// 3.7. The KW partial tiles are added in LDS in wave order before
 // the epilogue (small_reduce_store), so each element's summation order depends on K and KW
 // alone: the same for all four transpose layouts, aligned or not.
 // An MFMA rounds its sum once per product, so a long sum costs precision: the steps of a batch go into
@@ -534,38 +536,33 @@ gemm_small_kernel(GemmParams p) {
 #pragma unroll
         for (int j = 0; j < FN; ++j) c[i][j] = Ops::mma(af[i], bf[j], s, c[i][j]);
   };
-  auto batch = [&](int t0, auto part_c) {
-    constexpr bool PART = decltype(part_c)::value;  // fewer than U steps are left: the rest count as zeros
-    V af[U][FM], bf[U][FN];
+  auto batch = [&](int t0, auto count) {
+    constexpr int R = decltype(count)::value;  // K steps
+    V af[R][FM], bf[R][FN];
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int t = PART ? min(t0 + u, fe - 1) : t0 + u;
+    for (int u = 0; u < R; ++u) {
 #pragma unroll
-      for (int i = 0; i < FM; ++i) af[u][i] = frag(A, p.lda, !TA, va[i], t);
+      for (int i = 0; i < FM; ++i) af[u][i] = frag(A, p.lda, !TA, va[i], t0 + u);
 #pragma unroll
-      for (int j = 0; j < FN; ++j) bf[u][j] = frag(B, p.ldb, TB, vb[j], t);
+      for (int j = 0; j < FN; ++j) bf[u][j] = frag(B, p.ldb, TB, vb[j], t0 + u);
     }
     __builtin_amdgcn_sched_barrier(0);  // all loads before the first MFMA
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      if (PART && u > 0) {
-        const bool live = t0 + u < fe;
-#pragma unroll
-        for (int i = 0; i < FM; ++i)
-#pragma unroll
-          for (int e = 0; e < E; ++e) af[u][i][e] = live ? af[u][i][e] : T(0);
-#pragma unroll
-        for (int j = 0; j < FN; ++j)
-#pragma unroll
-          for (int e = 0; e < E; ++e) bf[u][j][e] = live ? bf[u][j][e] : T(0);
-      }
+    for (int u = 0; u < R; ++u) {
       multiply(af[u], bf[u], acc[u % NA]);
-      __builtin_amdgcn_sched_barrier(0);  // in the order of the loads
+      // in the order of the loads; the long sums of 16 waves gain more from steps side by side
+      if constexpr (KW < 16) __builtin_amdgcn_sched_barrier(0);
     }
   };
   int t0 = sb;
-  for (; t0 + U <= fe; t0 += U) batch(t0, std::false_type{});
-  if (t0 < fe) batch(t0, std::true_type{});
+  for (; t0 + U <= fe; t0 += U) batch(t0, std::integral_constant<int, U>{});
+  const int rest = fe - t0;
+  if (rest == 1) batch(t0, std::integral_constant<int, 1>{});
+  if constexpr (U > 2)
+    if (rest == 2) batch(t0, std::integral_constant<int, 2>{});
+  if constexpr (U > 3)
+    if (rest == 3) batch(t0, std::integral_constant<int, 3>{});
+  static_assert(U >= 2 && U <= 4, "rests of up to three steps");
   if (se > fe) multiply(ae, be, acc[NA - 1]);
 #pragma unroll
   for (int u = 1; u < NA; ++u)
