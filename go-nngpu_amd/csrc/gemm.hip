@@ -2162,6 +2162,10 @@ int launch_gemm(const GemmDesc &d, hipStream_t s, CError *err) {
     bool pack = !vec && big && !small && pack_bytes <= ((size_t)4 << 30) && pack_grid_y <= 65535;
     // A product of at most 64 rows (takes_rows), slices of K only outside graph capture (their
     // partial products take scratch) and where the scratch can be had.
+    if (takes_gemv(d, b_ok)) {
+      e = launch_gemv(d, s);
+      return e == hipSuccess ? 0 : hip_error(err, -6, "gemm launch", e);
+    }
     RowsPlan rows;
     if (d.M <= 64 && d.batch == 1 && plan_rows(d, true, &rows) && takes_rows(d, rows, a_ok, b_ok, small)) {
       std::unique_lock<std::mutex> lk;

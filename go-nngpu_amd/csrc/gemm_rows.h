@@ -18,4 +18,9 @@ bool plan_rows(const GemmDesc &d, bool split_ok, RowsPlan *out);
 // C with the epilogue (plan.S == 1) or the partial products of the slices into part.
 hipError_t launch_rows(const GemmDesc &d, const RowsPlan &plan, float *part, hipStream_t s);
 
+// Products of 1 to 4 rows with a wide W stored K x N and little K, W aligned (b_ok): gemv_nn_kernel. One
+// launch, no scratch.
+bool takes_gemv(const GemmDesc &d, bool b_ok);
+hipError_t launch_gemv(const GemmDesc &d, hipStream_t s);
+
 }  // namespace gn

@@ -266,6 +266,90 @@ __global__ void __launch_bounds__(KW * 64) gemm_rows_kernel(GemmParams p, int S)
   }
 }
 
+// ------------------------------------------------------------------ wide products of few k (GEMV)
+// C = act(alpha X W + beta C + bias) for X of R <= 4 rows, W stored K x N: lane l of a workgroup owns
+// columns n0 + E l .. + E - 1 (4 bytes of each row of W: 256 contiguous bytes by a wave); the KW waves
+// split K into contiguous ranges, summed with fmaf on the VALU, and the partials are added in LDS as a
+// tree (in wave order they lost more than the sums did). Bound by reading W, or, where W is short, by launch and the latency of one
+// round of loads: nothing else is on the path, where gemm_rows_kernel needs K for its pipeline (it takes
+// none below 256) and the tiled kernels 64 rows. us on MI355X, W in the caches (64 x 64 tiles or
+// gemm_rows_kernel -> this): fp32 1 x 32768 x 255 17.4 -> 4.9, 4 x 65536 x 128 13.1 -> 7.3, 1 x 16384 x 512
+// 5.4 -> 4.6; fp16 2 x 32768 x 128 5.4 -> 2.7, 1 x 65536 x 256 6.0 -> 4.2.
+template <typename T, int R, int E, int KW>
+__global__ void __launch_bounds__(KW * 64) gemv_nn_kernel(GemmParams p) {
+  __shared__ float red[KW][R][64 * E];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const long nb = (long)blockIdx.x * 64 * E, n0 = nb + (long)lane * E;
+  const T *__restrict__ W = static_cast<const T *>(p.B);
+  const T *__restrict__ X = static_cast<const T *>(p.A);
+  const long kb = p.K * wave / KW, ke = p.K * (wave + 1) / KW;
+  float acc[R][E];
+#pragma unroll
+  for (int m = 0; m < R; ++m)
+#pragma unroll
+    for (int e = 0; e < E; ++e) acc[m][e] = 0.0f;
+  if (n0 < p.N) {  // N is a multiple of E: the E columns are all inside or all past N
+    typedef typename VecOf<T, E>::type VE;
+    auto step = [&](long k) {
+      const VE w = *reinterpret_cast<const VE *>(W + k * p.ldb + n0);
+#pragma unroll
+      for (int m = 0; m < R; ++m) {
+        const float x = (float)X[m * p.lda + k];  // the same for the whole wave
+        if constexpr (E == 1) {
+          acc[m][0] = fmaf(x, (float)w, acc[m][0]);
+        } else {
+#pragma unroll
+          for (int e = 0; e < E; ++e) acc[m][e] = fmaf(x, (float)w[e], acc[m][e]);
+        }
+      }
+    };
+    long k = kb;
+    for (; k + 8 <= ke; k += 8) {
+#pragma unroll
+      for (int u = 0; u < 8; ++u) step(k + u);
+    }
+    for (; k < ke; ++k) step(k);
+  }
+#pragma unroll
+  for (int m = 0; m < R; ++m)
+#pragma unroll
+    for (int e = 0; e < E; ++e) red[wave][m][lane * E + e] = acc[m][e];
+  __syncthreads();
+  for (int o = threadIdx.x; o < R * 64 * E; o += KW * 64) {
+    const int m = o / (64 * E), c = o % (64 * E);
+    const long n = nb + c;
+    if (n >= p.N) continue;
+    float v[KW];
+#pragma unroll
+    for (int w = 0; w < KW; ++w) v[w] = red[w][m][c];
+#pragma unroll
+    for (int h = KW / 2; h > 0; h /= 2)
+#pragma unroll
+      for (int w = 0; w < h; ++w) v[w] += v[w + h];
+    float *dst = p.C + m * p.ldc + n;
+    const float old = p.beta != 0.0f ? *dst : 0.0f;
+    *dst = apply_act(p.act, p.alpha * v[0] + p.beta * old + (p.bias ? p.bias[n] : 0.0f), p.act_alpha);
+  }
+}
+
+template <typename T, int R>
+hipError_t launch_gemv_r(const GemmParams &p, hipStream_t s) {
+  constexpr int E = sizeof(T) == 2 ? 2 : 1;  // 4 bytes per lane and row of W
+  const unsigned grid = (unsigned)((p.N + 64 * E - 1) / (64 * E));
+  hipLaunchKernelGGL((gemv_nn_kernel<T, R, E, 16>), dim3(grid), dim3(1024), 0, s, p);
+  return hipGetLastError();
+}
+
+template <typename T>
+hipError_t launch_gemv_t(const GemmParams &p, hipStream_t s) {
+  switch (p.M) {
+    case 1: return launch_gemv_r<T, 1>(p, s);
+    case 2: return launch_gemv_r<T, 2>(p, s);
+    case 3: return launch_gemv_r<T, 3>(p, s);
+    default: return launch_gemv_r<T, 4>(p, s);
+  }
+}
+
 // ------------------------------------------------------------------ shapes
 // Shape fn: NT 16, 32 or 48 columns; NN fp32 16, 32 or 64, fp16 32 or 64 (FN values). Waves and
 // depths are the ones that measured best or within 3% of it: 16 waves of two steps for 16 NT columns
@@ -367,6 +451,28 @@ bool plan_rows(const GemmDesc &d, bool split_ok, RowsPlan *out) {
   if (out->us >= 1e30) return false;
   out->part_bytes = out->S > 1 ? (size_t)out->S * splitk_stride(d.M, d.N) * sizeof(float) : 0;
   return true;
+}
+
+// Where gemv_nn_kernel beat the other kernels on a grid of 1 to 4 rows, N 256 to 65536 and K 16 to 8192
+// (time over the best of theirs): K below 256 from N = 8192, 0.35-0.8 (N = 4096 0.9-1.2); fp32 to K = 1024
+// the further N is from M K (1 x 16384 x 1024 0.95, 2 x 11008 x 384 0.91; 2 x 8192 x 512 1.2, 4 rows 0.9-1.1
+// whatever the size), fp16 from N = 32768 (0.83-0.98; 16384 x 512 1.05-1.3).
+bool takes_gemv(const GemmDesc &d, bool b_ok) {
+  if (d.batch != 1 || d.ta || d.tb || d.M > 4 || !b_ok || d.N < 8192 || d.K > 1024 || d.N > (1L << 30)) return false;
+  if (d.K < 256) return true;
+  if (d.dtype == GN_F32) return d.M <= 3 && d.N >= 13 * d.M * d.K;
+  return d.N >= (d.K < 384 ? 5120 * d.M : 32768);
+}
+
+hipError_t launch_gemv(const GemmDesc &d, hipStream_t s) {
+  GemmParams p{};
+  p.A = d.A; p.B = d.B; p.C = d.C;
+  p.M = d.M; p.N = d.N; p.K = d.K;
+  p.lda = d.lda; p.ldb = d.ldb; p.ldc = d.ldc;
+  p.alpha = d.alpha; p.beta = d.beta;
+  p.bias = d.bias;
+  p.act = d.act; p.act_alpha = d.act_alpha;
+  return d.dtype == GN_F16 ? launch_gemv_t<_Float16>(p, s) : launch_gemv_t<float>(p, s);
 }
 
 hipError_t launch_rows(const GemmDesc &d, const RowsPlan &plan, float *part, hipStream_t s) {

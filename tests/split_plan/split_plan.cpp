@@ -12,12 +12,14 @@
 // others of the same launch read, and whichever kernel finds a value stops the reduce and calls for the
 // fp32 kernels, for this call only.
 // Exit 0: no violation; 1: violations. Prints how many cuts of each form it saw. With arguments M N K
-// batch layout gap (nn, nt, tn or tt; gap: elements between the batches' B) it prints that product's cut.
+// batch layout gap (nn, nt, tn or tt; gap: elements between the batches' B) it prints that product's cut;
+// with route f32|f16 layout M N K, the few-rows kernel that takes that product (aligned operands).
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <vector>
 
+#include "../../go-nngpu_amd/csrc/gemm_rows.h"
 #include "../../go-nngpu_amd/csrc/gemm_split.h"
 
 using namespace gn;
@@ -103,6 +105,12 @@ static_assert(split_fp32_needed({kSeq, kOld}, kSeq) && split_fp32_needed({kOld, 
 static_assert(!split_fp32_needed({kOld, kOld}, kSeq), "an earlier call's values");
 
 int main(int argc, char **argv) {
+  if (argc == 7 && std::strcmp(argv[1], "route") == 0) {
+    GemmDesc d = product(std::atol(argv[4]), std::atol(argv[5]), std::atol(argv[6]), 1, argv[3][0] == 't', argv[3][1] == 't', 0);
+    d.dtype = argv[2][1] == '3' ? GN_F32 : GN_F16;
+    std::printf("%s\n", takes_gemv(d, true) ? "gemv" : "-");
+    return 0;
+  }
   if (argc == 7) {
     const GemmDesc d = product(std::atol(argv[1]), std::atol(argv[2]), std::atol(argv[3]), std::atol(argv[4]),
                                argv[5][0] == 't', argv[5][1] == 't', std::atol(argv[6]));

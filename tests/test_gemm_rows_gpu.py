@@ -127,3 +127,33 @@ def test_rows_infinity_stays_in_its_row_and_column(dev, layout):
     assert torch.equal(torch.isnan(c), torch.isnan(ref)) and torch.equal(torch.isinf(c), torch.isinf(ref))
     fine = torch.isfinite(ref)
     assert _rel(c[fine], ref[fine]) <= 1e-5
+
+
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("M,N,K", [(1, 8192, 1), (2, 8200, 15), (3, 8256, 16), (4, 11008, 31), (1, 16384, 130), (4, 8192, 200), (2, 32776, 255),
+                                   (3, 10008, 256), (2, 32768, 401), (1, 65536, 1024)])
+def test_rows_wide_with_little_k(dev, M, N, K, half):
+    """X W of 1-4 rows and few k (gemv_nn_kernel): fewer k than waves, whole rounds of eight and a rest, columns past the
+    last workgroup's, padded leading dimensions; an infinity stays in its row and column."""
+    import torch
+
+    g = torch.Generator(device=dev).manual_seed(M + 3 * N + 5 * K)
+    dt = torch.float16 if half else torch.float32
+    bias = torch.randn((N,), generator=g, device=dev)
+    c0 = torch.randn((M, N), generator=g, device=dev)
+    for pad in (0, 8):
+        x = _operand(torch, g, dev, M, K, K + pad, dt)
+        w = _operand(torch, g, dev, K, N, N + pad, dt, 0.05)
+        ref = x.double() @ w.double().contiguous()
+        c = torch.full((M, N + 3), float("nan"), device=dev)[:, :N]
+        print("wide", M, N, K, half, pad, flush=True)
+        G.gemm(x, w, c, bias=bias, act=G.ACT_RELU)
+        assert _rel(c, (ref + bias.double()).clamp_min(0.0)) <= 3e-7  # K <= 1024: chains of 64 and a tree of 16, 1.5e-7
+        y = c0.clone()
+        G.gemm(x, w, y, alpha=-0.5, beta=2.0)
+        assert _rel(y, -0.5 * ref + 2.0 * c0.double()) <= 3e-7
+    x[M - 1, K - 1] = float("inf")
+    w[K - 1, N - 1] = float("nan")
+    G.gemm(x, w, c)
+    ref = x.double() @ w.double().contiguous()
+    assert torch.equal(torch.isnan(c), torch.isnan(ref)) and torch.equal(torch.isinf(c), torch.isinf(ref))

@@ -45,3 +45,19 @@ def test_gpu_cases_reach_the_cuts_they_name(plan, M, N, K, batch, layout, gap, f
     nb, kc, raw, S = map(int, m.groups())
     assert {"batch": 1 < nb < batch, "single": nb == 1 < batch, "k": kc < K}[form.split("-")[0]]
     assert raw == form.endswith("raw")
+
+
+# Products whose time a kernel of their own brings down: dtype, layout, M, N, K, kernel (on MI355X the next best took
+# the factor in the comment)
+ROUTES = [("f32", "nn", 1, 32768, 255, "gemv"),  # 3.5
+          ("f32", "nn", 4, 65536, 128, "gemv"),  # 1.8
+          ("f16", "nn", 2, 32768, 128, "gemv"),  # 2.0
+          ("f32", "nn", 1, 16384, 512, "gemv"),  # 1.17
+          ("f16", "nn", 1, 65536, 256, "gemv"),  # 1.4
+          ]
+
+
+@pytest.mark.parametrize("dtype,layout,M,N,K,kernel", ROUTES)
+def test_few_rows_take_the_kernel_that_measured_best(plan, dtype, layout, M, N, K, kernel):
+    out = subprocess.run([plan, "route", dtype, layout, str(M), str(N), str(K)], capture_output=True, text=True).stdout
+    assert out.strip() == kernel
