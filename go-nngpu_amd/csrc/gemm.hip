@@ -1991,24 +1991,6 @@ hipError_t dispatch_behind(bool ta, bool tb, const GemmParams &p, long batch, hi
   return tb ? launch_f32_behind<false, true, VEC>(p, batch, s) : launch_f32_behind<false, false, VEC>(p, batch, s);
 }
 
-// Where gemm_rows.hip takes a product it can (plan_rows). Up to 16 rows: always, but for what the
-// small-product kernel takes with W below 2^20 elements (1 x 1000 x 1000 fp16 3.8 us against 2.9
-// there). Up to 32 from 2^20 elements of W, in fp16 below 2^25 (28 rows x 11008 x 4096: 28.9 us
-// against 27.7 on the split-K ring); up to 64 in fp16 from 2^20 to 12 M elements (at 16 M level,
-// at 45 M 36 against 30), both fp16 ones only past the small-product kernel's range (64 x 1024 x
-// 1024: 7.2 us against 4.5), in fp32 by price (the fp32 tiles' is for a
-// warm W and 15% low with W from HBM: 40 x 11008 x 4096 74 -> 59), and instead of the small-product
-// kernel for K of 2048 and more (32 x 2048 x 1024: 7.4 us against 5.2; 64 x 256 x 4096: 17.2 -> 11.3 us; 64 x 512 x 512: 8.1 against 5.0).
-bool takes_rows(const GemmDesc &d, const RowsPlan &rows, bool a_ok, bool b_ok, bool small) {
-  const double w = (double)d.N * (double)d.K;
-  if (small && w < (double)(1L << 20)) return false;
-  if (d.M <= 16) return true;
-  if (w < (double)(1L << 20)) return false;
-  if (d.dtype == GN_F16) return !small && w < (d.M <= 32 ? (double)(1L << 25) : 12.0e6);
-  if (small) return d.K >= 2048;
-  return d.M <= 32 || rows.us < 1.15 * (f32_cores_us(d, a_ok, b_ok) + 3.0);
-}
-
 // Enqueues the product by `cut` with ws (cut.ws_bytes) as its workspace. Behind every part's split
 // kernels the fp32 kernels are enqueued too; they return at once unless an operand holds a value the
 // split does not (an infinity, a NaN, or 2^36 and more), in which case they compute C, or the partial
@@ -2061,6 +2043,44 @@ hipError_t run_split(const GemmDesc &d, const SplitCut &cut, bool vec, char *ws,
 }
 
 }  // namespace
+
+bool takes_small(const GemmDesc &d, bool vec) {
+  return small_offsets_fit(d.lda, d.ldb) && (d.dtype == GN_F32 ? f32_small_tile(d.M, d.N, d.K, d.batch, d.ta, d.tb)
+                                                               : f16_small_tile(d.M, d.N, d.K, d.batch, d.ta, d.tb, vec)) != 0;
+}
+
+// Where gemm_rows.hip takes a product it can (plan_rows): nearly everywhere up to 16 rows, less and less
+// beyond. Each exception below is where the kernels that take the product instead (the small-product
+// kernel, or the tiles with or without slices of K) measured faster on a grid of 1 to 64 rows, K 256 to
+// 8192 and N 256 to 65536, W warm and from HBM; in brackets the time here over theirs.
+bool takes_rows(const GemmDesc &d, const RowsPlan &rows, bool a_ok, bool b_ok, bool small) {
+  const double w = (double)d.N * (double)d.K;
+  const bool f16 = d.dtype == GN_F16, nt = d.tb;
+  const long M = d.M, N = d.N, K = d.K;
+  if (small && w < (double)(1L << 20)) return false;  // [1 x 1000 x 1000 fp16 1.3]
+  if (!small && !f16 && N < 512 && K > 4096) return false;  // 8 slices of 16 tiles at most [64 x 256 x 8192 1.35]
+  if (M <= 16) {
+    if (!f16) return true;
+    if (!nt) return !(M > 4 && N >= 65536 && K >= 512);  // [8 x 65536 x 2048 1.11]
+    if (small && K <= 2048) return N > 2048 && N < 8192 && (M > 4 || (M > 1 && K > 1024 && N > 4096));  // [1 x 5000 x 1024 1.2, 2 x 11008 x 2048 1.26, 8 x 1024 x 1024 1.05]
+    if (small && M <= 4 && N >= 8192 && (K <= 4096 || N == 8192)) return false;  // [2 x 11008 x 4096 1.14]
+    return !(M > 4 && N >= 65536 && K >= 512 && K <= 1024);  // [16 x 65536 x 512 1.3]
+  }
+  if (w < (double)(1L << 20)) return false;
+  if (f16) {
+    // NN past 64 tiles of 64 x 64 it is faster than the small-product kernel too [64 x 5000 x 1024 0.6]
+    if (small && (nt || N <= 4096)) return false;  // [64 x 1024 x 1024 1.6]
+    if (N >= 32768 || w >= (M <= 32 ? (double)(1L << 25) : 12.0e6)) return false;  // [32 x 32768 x 512 1.33, 64 x 11008 x 4096 1.2]
+    if (K < 512 && (M > 32 ? N > 8192 || (nt && M > 48 && N == 8192) : nt && N > 8192 && N < 16384)) return false;  // [64 x 11008 x 256 1.4]
+    return !(nt && (M > 32 ? N >= 16384 : M > 24 && K >= 4096 && N > 4096));  // [64 x 16384 x 512 1.09, 32 x 5000 x 4096 1.16]
+  }
+  // up to 32 rows from K = 2048; beyond only where there is more to read, or little N [64 x 512 x 2048 1.1-1.3]
+  if (small) return K >= 2048 && (M <= 32 || w >= (double)(1L << 22) || K >= 16 * N);  // [32 x 2048 x 1024 1.4, 64 x 512 x 512 1.6]
+  if (N > 8192 && K <= (M > 48 ? 1023 : M > 32 ? (N < 16384 ? 511 : 512) : nt ? 0 : 511)) return false;  // [64 x 11008 x 256 NN 1.5, 32 x 16384 x 256 NN 1.1]
+  if (nt && N >= 32768 && K < 4096) return false;  // [32 x 32768 x 512 1.26]
+  // the fp32 tiles' price is for a warm W and 15% low with W from HBM: 40 x 11008 x 4096 74 -> 59 us
+  return M <= 32 || rows.us < 1.15 * (f32_cores_us(d, a_ok, b_ok) + 3.0);
+}
 
 // true when the product runs on the bf16 matrix cores: priced (the operands' packing, the
 // product, the reduce, 3 us for the fp32 kernels that stand behind it) at least 7% below the
@@ -2156,9 +2176,7 @@ int launch_gemm(const GemmDesc &d, hipStream_t s, CError *err) {
         (size_t)((a_ok ? 0 : d.M) + (b_ok ? 0 : d.N)) * (size_t)Kp * esz * (size_t)std::min(kMaxZ, d.batch);
     const bool big = (double)d.M * d.N * d.K >= (double)(1L << 24);
     const long pack_grid_y = (a_ok ? 0 : (d.M + 63) / 64) + (b_ok ? 0 : (d.N + 63) / 64);
-    const bool small = small_offsets_fit(d.lda, d.ldb) &&
-                       (d.dtype == GN_F32 ? f32_small_tile(d.M, d.N, d.K, d.batch, d.ta, d.tb)
-                                          : f16_small_tile(d.M, d.N, d.K, d.batch, d.ta, d.tb, vec)) != 0;
+    const bool small = takes_small(d, vec);
     bool pack = !vec && big && !small && pack_bytes <= ((size_t)4 << 30) && pack_grid_y <= 65535;
     // A product of at most 64 rows (takes_rows), slices of K only outside graph capture (their
     // partial products take scratch) and where the scratch can be had.

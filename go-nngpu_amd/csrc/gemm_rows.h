@@ -10,6 +10,7 @@ namespace gn {
 // the slices' partial products.
 struct RowsPlan {
   int fn = 0, S = 1;
+  bool few = false;  // NT, fn 1: 4 waves per workgroup
   double us = 0;
   size_t part_bytes = 0;
 };
@@ -22,5 +23,10 @@ hipError_t launch_rows(const GemmDesc &d, const RowsPlan &plan, float *part, hip
 // launch, no scratch.
 bool takes_gemv(const GemmDesc &d, bool b_ok);
 hipError_t launch_gemv(const GemmDesc &d, hipStream_t s);
+// Whether the small-product kernel takes a product if no other does before it (gemm.hip). vec: the operands suit 16-byte
+// vectors.
+bool takes_small(const GemmDesc &d, bool vec);
+// Whether launch_rows takes a product that plan_rows has planned (gemm.hip). small: takes_small.
+bool takes_rows(const GemmDesc &d, const RowsPlan &rows, bool a_ok, bool b_ok, bool small);
 
 }  // namespace gn

@@ -353,7 +353,8 @@ hipError_t launch_gemv_t(const GemmParams &p, hipStream_t s) {
 // ------------------------------------------------------------------ shapes
 // Shape fn: NT 16, 32 or 48 columns; NN fp32 16, 32 or 64, fp16 32 or 64 (FN values). Waves and
 // depths are the ones that measured best or within 3% of it: 16 waves of two steps for 16 NT columns
-// (8 with 33-64 rows, which need the registers), 4 waves for the widest NN shapes.
+// (8 with 33-64 rows, which need the registers; 4 where plan_rows says so), 4 waves for the widest NN
+// shapes.
 template <typename T, bool TB, int FM, int FN, int KW, int D, bool XV, int H = 2>
 hipError_t launch_shape(const GemmParams &p, int S, hipStream_t s) {
   const dim3 grid((unsigned)((p.N + 16 * FN - 1) / (16 * FN)), 1, (unsigned)S);
@@ -374,8 +375,10 @@ hipError_t launch_nn(const GemmParams &p, int fn, int S, hipStream_t s) {
 }
 
 template <typename T, int FM>
-hipError_t launch_fm(const GemmParams &p, bool tb, bool xv, int fn, int S, hipStream_t s) {
+hipError_t launch_fm(const GemmParams &p, bool tb, bool xv, int fn, bool few, int S, hipStream_t s) {
   if (tb) {
+    if constexpr (FM == 1)
+      if (few) return launch_shape<T, true, 1, 1, 4, 2, true>(p, S, s);
     if (fn == 1) return launch_shape<T, true, FM, 1, FM <= 2 ? 16 : 8, 2, true>(p, S, s);
     if (fn == 2) return launch_shape<T, true, FM, 2, 8, 2, true>(p, S, s);
     return launch_shape<T, true, FM, 3, 8, 2, true>(p, S, s);
@@ -386,12 +389,12 @@ hipError_t launch_fm(const GemmParams &p, bool tb, bool xv, int fn, int S, hipSt
 }
 
 template <typename T>
-hipError_t launch_rows_t(const GemmParams &p, bool tb, bool xv, int fn, int S, hipStream_t s) {
+hipError_t launch_rows_t(const GemmParams &p, bool tb, bool xv, int fn, bool few, int S, hipStream_t s) {
   switch ((p.M + 15) / 16) {
-    case 1: return launch_fm<T, 1>(p, tb, xv, fn, S, s);
-    case 2: return launch_fm<T, 2>(p, tb, xv, fn, S, s);
-    case 3: return launch_fm<T, 3>(p, tb, xv, fn, S, s);
-    default: return launch_fm<T, 4>(p, tb, xv, fn, S, s);
+    case 1: return launch_fm<T, 1>(p, tb, xv, fn, few, S, s);
+    case 2: return launch_fm<T, 2>(p, tb, xv, fn, few, S, s);
+    case 3: return launch_fm<T, 3>(p, tb, xv, fn, few, S, s);
+    default: return launch_fm<T, 4>(p, tb, xv, fn, few, S, s);
   }
 }
 
@@ -449,6 +452,16 @@ bool plan_rows(const GemmDesc &d, bool split_ok, RowsPlan *out) {
     }
   }
   if (out->us >= 1e30) return false;
+  // Many NT tiles of 16 columns with little K each: of 16 waves most have no step or one, and two
+  // workgroups of them fill a CU, which then waits out one round of loads after another; eight of 4
+  // waves do so at a time (16 waves -> 4, warm: fp16 1 x 65536 x 256 22.8 -> 7.2 us, 2 x 32768 x 512 11.3 -> 5.8,
+  // 8 x 16384 x 1024 13.6 -> 9.8; fp32 1 x 32768 x 256 14.3 -> 7.2). With more K or rows level or slower
+  // (fp16 16 x 16384 x 1024 9.4 -> 11.1).
+  out->few = d.tb && d.N >= 4096 &&
+             (f16 ? (d.K < 512 && (d.M <= 12 || (d.M <= 16 && (d.N < 16384 || d.N >= 65536)))) || (d.K < 1024 && d.M <= 8) || (d.K <= 1024 && (d.M <= 2 || (d.M <= 8 && d.N >= 8192)))
+                  : (d.K < 512 && (d.M <= 4 || (d.M <= 8 && d.N >= 8192))) || (d.M <= 4 && d.N > 8192 && d.K < 1024) ||
+                        (d.M <= 2 && d.N >= 16384 && d.K >= 2048 && d.K < 4096));
+  if (out->few) out->fn = 1, out->S = 1;
   out->part_bytes = out->S > 1 ? (size_t)out->S * splitk_stride(d.M, d.N) * sizeof(float) : 0;
   return true;
 }
@@ -494,8 +507,8 @@ hipError_t launch_rows(const GemmDesc &d, const RowsPlan &plan, float *part, hip
     p.act = -1;
   }
   const bool xv = x_vectors(d);
-  return d.dtype == GN_F16 ? launch_rows_t<_Float16>(p, d.tb, xv, plan.fn, plan.S, s)
-                           : launch_rows_t<float>(p, d.tb, xv, plan.fn, plan.S, s);
+  return d.dtype == GN_F16 ? launch_rows_t<_Float16>(p, d.tb, xv, plan.fn, plan.few, plan.S, s)
+                           : launch_rows_t<float>(p, d.tb, xv, plan.fn, plan.few, plan.S, s);
 }
 
 }  // namespace gn

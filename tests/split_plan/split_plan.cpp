@@ -13,7 +13,7 @@
 // fp32 kernels, for this call only.
 // Exit 0: no violation; 1: violations. Prints how many cuts of each form it saw. With arguments M N K
 // batch layout gap (nn, nt, tn or tt; gap: elements between the batches' B) it prints that product's cut;
-// with route f32|f16 layout M N K, the few-rows kernel that takes that product (aligned operands).
+// with route f32|f16 layout M N K, the kernel that takes that product (aligned operands).
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -108,7 +108,11 @@ int main(int argc, char **argv) {
   if (argc == 7 && std::strcmp(argv[1], "route") == 0) {
     GemmDesc d = product(std::atol(argv[4]), std::atol(argv[5]), std::atol(argv[6]), 1, argv[3][0] == 't', argv[3][1] == 't', 0);
     d.dtype = argv[2][1] == '3' ? GN_F32 : GN_F16;
-    std::printf("%s\n", takes_gemv(d, true) ? "gemv" : "-");
+    const bool small = takes_small(d, true);
+    RowsPlan rows;
+    if (takes_gemv(d, true)) std::printf("gemv\n");
+    else if (plan_rows(d, true, &rows) && takes_rows(d, rows, true, true, small)) std::printf("rows%s\n", rows.few ? "-4" : "");
+    else std::printf("%s\n", small ? "small" : "tiles");
     return 0;
   }
   if (argc == 7) {

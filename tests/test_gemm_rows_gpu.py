@@ -157,3 +157,29 @@ def test_rows_wide_with_little_k(dev, M, N, K, half):
     G.gemm(x, w, c)
     ref = x.double() @ w.double().contiguous()
     assert torch.equal(torch.isnan(c), torch.isnan(ref)) and torch.equal(torch.isinf(c), torch.isinf(ref))
+
+
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("M,N,K", [(1, 4096, 256), (2, 65536, 264), (8, 16400, 520), (12, 5001, 400), (16, 8192, 504), (4, 11008, 1016), (1, 8199, 1024),
+                                   (2, 16384, 2048), (3, 9000, 328)])
+def test_rows_four_waves(dev, M, N, K, half):
+    """X W^T on tiles of 16 columns with 4 waves (plan_rows): waves with no whole step, one, and several
+    with a rest; a ragged last tile; padded leading dimensions."""
+    import torch
+
+    g = torch.Generator(device=dev).manual_seed(M + 3 * N + 5 * K)
+    dt = torch.float16 if half else torch.float32
+    bias = torch.randn((N,), generator=g, device=dev)
+    for pad in (0, 8):
+        x = _operand(torch, g, dev, M, K, K + pad, dt)
+        w = _operand(torch, g, dev, N, K, K + pad, dt, 0.05)
+        ref = x.double() @ w.t().double().contiguous()
+        c = torch.full((M, N + 3), float("nan"), device=dev)[:, :N]
+        print("four waves", M, N, K, half, pad, flush=True)
+        G.gemm(x, w, c, transB=True, bias=bias, act=G.ACT_RELU)
+        assert _rel(c, (ref + bias.double()).clamp_min(0.0)) <= 1e-6
+    x[M - 1, K - 1] = float("inf")
+    w[N - 1, 0] = float("nan")
+    G.gemm(x, w, c, transB=True)
+    ref = x.double() @ w.t().double().contiguous()
+    assert torch.equal(torch.isnan(c), torch.isnan(ref)) and torch.equal(torch.isinf(c), torch.isinf(ref))

@@ -54,7 +54,19 @@ ROUTES = [("f32", "nn", 1, 32768, 255, "gemv"),  # 3.5
           ("f16", "nn", 2, 32768, 128, "gemv"),  # 2.0
           ("f32", "nn", 1, 16384, 512, "gemv"),  # 1.17
           ("f16", "nn", 1, 65536, 256, "gemv"),  # 1.4
-          ]
+          ("f16", "nt", 1, 65536, 256, "rows-4"),  # 3.2 (16 waves)
+          ("f16", "nt", 8, 32768, 512, "rows-4"),  # 1.7 (16 waves)
+          ("f32", "nt", 2, 32768, 256, "rows-4"),  # 1.9 (16 waves)
+          ("f16", "nt", 2, 11008, 4096, "small"),  # 1.14 (rows)
+          ("f16", "nt", 1, 16384, 2048, "small"),  # 1.3 (rows)
+          ("f16", "nt", 1, 1024, 1024, "small"),  # 1.05 (rows)
+          ("f16", "nt", 32, 32768, 512, "tiles"),  # 1.33 (rows)
+          ("f32", "nt", 64, 11008, 256, "tiles"),  # 1.17 (rows)
+          ("f32", "nn", 64, 16384, 512, "tiles"),  # 1.16 (rows)
+          ("f32", "nt", 64, 256, 8192, "tiles"),  # 1.35 (rows)
+          ("f32", "nn", 64, 512, 2048, "small"),  # 1.29 (rows)
+          ("f32", "nt", 16, 11008, 4096, "rows"), ("f16", "nn", 4, 11008, 4096, "rows"), ("f32", "nn", 64, 256, 4096, "rows"),
+          ("f16", "nn", 64, 5000, 1024, "rows")]  # 1.3, 1.35, 1.5, 1.7 (small or tiles)
 
 
 @pytest.mark.parametrize("dtype,layout,M,N,K,kernel", ROUTES)
