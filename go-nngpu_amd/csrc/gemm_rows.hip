@@ -65,8 +65,15 @@ struct VecOf<float, 1> {
 
 // Steps of H substeps; XV: X's rows allow 16-byte loads. Rows past M and columns past N are
 // clamped to the last ones (loaded, multiplied and not stored). NN: N and ldb are multiples of FN.
+// NA: sums per element and wave; the substeps in flight take them in turn. An MFMA rounds its sum
+// once per product, and where 4 or 8 waves share K one sum each lost up to half the precision the tiled
+// kernels have in NN: fp32 4 x 11008 x 4096 5.7e-7 against 2.9e-7 relative to float64, now 2.9e-7 in the
+// same time. FLUSH: with 17 to 32 rows there are no registers for that (28 spilled; two sums in AGPRs cost
+// 10-20%), and the sum of each round of loads is added to a total instead (with fewer rows, or in the
+// 8-wave shapes, that cost up to 20% where K is short).
 template <typename T, bool TB, int FM, int FN, int KW, int D, int H, bool XV>
-__global__ void __launch_bounds__(KW * 64) gemm_rows_kernel(GemmParams p, int S) {
+__global__ void __launch_bounds__(KW * 64) __attribute__((amdgpu_waves_per_eu(KW > 8 ? KW / 4 : FM > 2 && KW == 4 ? 1 : 2)))
+gemm_rows_kernel(GemmParams p, int S) {
   typedef RowOps<T> Ops;
   typedef typename Ops::V V;
   constexpr int E = Ops::E, KS = Ops::KS, STEP = KS * H, BN = 16 * FN;
@@ -113,13 +120,25 @@ __global__ void __launch_bounds__(KW * 64) gemm_rows_kernel(GemmParams p, int S)
       for (int m = 0; m < FM; ++m) x[d][h][m] = load_x(xp[m] + k + h * KS);
     }
   };
-  float4_t acc[FM][FN];
+  constexpr int NA = FM > 1 || KW > 8 || (TB && (KW == 8 || sizeof(T) == 2)) ? 1 : !TB && KW == 4 && sizeof(T) == 4 ? 4 : 2;
+  constexpr bool FLUSH = FM == 2 && KW == 4 && sizeof(T) == 4;
+  static_assert(D * H % NA == 0, "the sums in turn");
+  float4_t acc[NA][FM][FN];
 #pragma unroll
-  for (int m = 0; m < FM; ++m)
+  for (int q = 0; q < NA; ++q)
 #pragma unroll
-    for (int n = 0; n < FN; ++n) acc[m][n] = float4_t{0.f, 0.f, 0.f, 0.f};
+    for (int m = 0; m < FM; ++m)
+#pragma unroll
+      for (int n = 0; n < FN; ++n) acc[q][m][n] = float4_t{0.f, 0.f, 0.f, 0.f};
+  float4_t flushed[FLUSH ? FM : 1][FLUSH ? FN : 1];
+  if constexpr (FLUSH) {
+#pragma unroll
+    for (int m = 0; m < FM; ++m)
+#pragma unroll
+      for (int n = 0; n < FN; ++n) flushed[m][n] = float4_t{0.f, 0.f, 0.f, 0.f};
+  }
   // B fragments of a substep: NT as loaded; NN fp32: register n of row j; NN fp16: the 8 rows' column n
-  auto mul = [&](const V (&xs)[FM], const WV (&ws)[NW]) {
+  auto mul = [&](const V (&xs)[FM], const WV (&ws)[NW], float4_t (&c)[FM][FN]) {
     V b[FN];
     if constexpr (TB) {
 #pragma unroll
@@ -161,7 +180,7 @@ __global__ void __launch_bounds__(KW * 64) gemm_rows_kernel(GemmParams p, int S)
 #pragma unroll
       for (int m = 0; m < FM; ++m)
 #pragma unroll
-        for (int n = 0; n < FN; ++n) acc[m][n] = Ops::mma(xs[m], b[n], s, acc[m][n]);
+        for (int n = 0; n < FN; ++n) c[m][n] = Ops::mma(xs[m], b[n], s, c[m][n]);
   };
   // the slice's whole steps [s0, s1); wave w takes s0 + w, s0 + w + KW, ...
   const long full = p.K / STEP, s0 = full * z / S, s1 = full * (z + 1) / S;
@@ -176,22 +195,28 @@ __global__ void __launch_bounds__(KW * 64) gemm_rows_kernel(GemmParams p, int S)
 #pragma unroll
       for (int d = 0; d < D; ++d) {
 #pragma unroll
-        for (int h = 0; h < H; ++h) mul(x[d][h], w[d][h]);
+        for (int h = 0; h < H; ++h) mul(x[d][h], w[d][h], acc[(d * H + h) % NA]);
         load(d, k + (t + d) * KW * STEP);
         __builtin_amdgcn_sched_barrier(0);
+      }
+      if constexpr (FLUSH) {
+#pragma unroll
+        for (int m = 0; m < FM; ++m)
+#pragma unroll
+          for (int n = 0; n < FN; ++n) flushed[m][n] = flushed[m][n] + acc[0][m][n], acc[0][m][n] = float4_t{0.f, 0.f, 0.f, 0.f};
       }
     }
 #pragma unroll
     for (int d = 0; d < D; ++d) {
 #pragma unroll
-      for (int h = 0; h < H; ++h) mul(x[d][h], w[d][h]);
+      for (int h = 0; h < H; ++h) mul(x[d][h], w[d][h], acc[(d * H + h) % NA]);
       if (t + d < mine) load(d, k + (t + d) * KW * STEP);
     }
 #pragma unroll
     for (int d = 0; d < D; ++d)
       if (t + d < mine) {
 #pragma unroll
-        for (int h = 0; h < H; ++h) mul(x[d][h], w[d][h]);
+        for (int h = 0; h < H; ++h) mul(x[d][h], w[d][h], acc[(d * H + h) % NA]);
       }
   } else {
 #pragma unroll
@@ -201,7 +226,7 @@ __global__ void __launch_bounds__(KW * 64) gemm_rows_kernel(GemmParams p, int S)
     for (int d = 0; d < D; ++d)
       if (d < mine) {
 #pragma unroll
-        for (int h = 0; h < H; ++h) mul(x[d][h], w[d][h]);
+        for (int h = 0; h < H; ++h) mul(x[d][h], w[d][h], acc[(d * H + h) % NA]);
       }
   }
   // the last K % STEP: substep by substep, elements at or past K zero in both operands
@@ -230,13 +255,19 @@ __global__ void __launch_bounds__(KW * 64) gemm_rows_kernel(GemmParams p, int S)
           if (kl + j < p.K) ws[j] = *reinterpret_cast<const WV *>(wp[0] + (kb + j) * p.ldb);
         }
       }
-      mul(xs, ws);
+      mul(xs, ws, acc[NA - 1]);
     }
   }
 #pragma unroll
   for (int m = 0; m < FM; ++m)
 #pragma unroll
-    for (int n = 0; n < FN; ++n) red[wave][m * FN + n][lane] = acc[m][n];
+    for (int n = 0; n < FN; ++n) {
+      float4_t v = acc[0][m][n];
+#pragma unroll
+      for (int q = 1; q < NA; ++q) v = v + acc[q][m][n];
+      if constexpr (FLUSH) v = v + flushed[m][n];
+      red[wave][m * FN + n][lane] = v;
+    }
   __syncthreads();
   for (int f = wave; f < FM * FN; f += KW) {
     float4_t v = red[0][f][lane];

@@ -183,3 +183,19 @@ def test_rows_four_waves(dev, M, N, K, half):
     G.gemm(x, w, c, transB=True)
     ref = x.double() @ w.t().double().contiguous()
     assert torch.equal(torch.isnan(c), torch.isnan(ref)) and torch.equal(torch.isinf(c), torch.isinf(ref))
+
+
+@pytest.mark.parametrize("layout,M,N,K", [("nn", 4, 11008, 4096), ("nn", 1, 16384, 8192), ("nn", 32, 11008, 8192), ("nn", 16, 5000, 8192),
+                                          ("nn", 2, 11008, 2400)])
+def test_rows_sum_k_in_short_chains(dev, layout, M, N, K):
+    """fp32: an MFMA rounds its sum once per product; chains of c products are off by about 2.5e-8 sqrt(c / 2) of
+    the result (the rms of a rounding, times the growth of the sum). Chains of at most K / 16 products, and
+    a sixth for adding them: 3.3e-7 at K = 4096, as the tiled kernels' (2.9e-7). One chain for each of 4
+    waves was 5.7e-7 off there."""
+    import torch
+
+    g = torch.Generator(device=dev).manual_seed(K)
+    x, w = torch.randn((M, K), generator=g, device=dev), torch.randn((K, N), generator=g, device=dev)
+    c = torch.empty((M, N), device=dev)
+    G.gemm(x, w.t().contiguous() if layout == "nt" else w, c, transB=layout == "nt")
+    assert _rel(c, x.double() @ w.double()) <= 7.0 / 6.0 * 2.5e-8 * (K / 32) ** 0.5
