@@ -2060,7 +2060,7 @@ bool takes_rows(const GemmDesc &d, const RowsPlan &rows, bool a_ok, bool b_ok, b
   if (small && w < (double)(1L << 20)) return false;  // [1 x 1000 x 1000 fp16 1.3]
   if (!small && !f16 && N < 512 && K > 4096) return false;  // 8 slices of 16 tiles at most [64 x 256 x 8192 1.35]
   if (M <= 16) {
-    if (!f16) return true;
+    if (!f16) return !(nt && small && M <= 4 && N >= 16384 && K < 4096);  // [1 x 32768 x 2048, W from HBM, 1.25; warm 0.9]
     if (!nt) return !(M > 4 && N >= 65536 && K >= 512);  // [8 x 65536 x 2048 1.11]
     if (small && K <= 2048) return N > 2048 && N < 8192 && (M > 4 || (M > 1 && K > 1024 && N > 4096));  // [1 x 5000 x 1024 1.2, 2 x 11008 x 2048 1.26, 8 x 1024 x 1024 1.05]
     if (small && M <= 4 && N >= 8192 && (K <= 4096 || N == 8192)) return false;  // [2 x 11008 x 4096 1.14]

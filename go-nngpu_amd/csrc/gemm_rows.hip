@@ -490,8 +490,7 @@ bool plan_rows(const GemmDesc &d, bool split_ok, RowsPlan *out) {
   // (fp16 16 x 16384 x 1024 9.4 -> 11.1).
   out->few = d.tb && d.N >= 4096 &&
              (f16 ? (d.K < 512 && (d.M <= 12 || (d.M <= 16 && (d.N < 16384 || d.N >= 65536)))) || (d.K < 1024 && d.M <= 8) || (d.K <= 1024 && (d.M <= 2 || (d.M <= 8 && d.N >= 8192)))
-                  : (d.K < 512 && (d.M <= 4 || (d.M <= 8 && d.N >= 8192))) || (d.M <= 4 && d.N > 8192 && d.K < 1024) ||
-                        (d.M <= 2 && d.N >= 16384 && d.K >= 2048 && d.K < 4096));
+                  : (d.K < 512 && (d.M <= 4 || (d.M <= 8 && d.N >= 8192))) || (d.M <= 4 && d.N > 8192 && d.K < 1024));
   if (out->few) out->fn = 1, out->S = 1;
   out->part_bytes = out->S > 1 ? (size_t)out->S * splitk_stride(d.M, d.N) * sizeof(float) : 0;
   return true;

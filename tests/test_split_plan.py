@@ -60,6 +60,7 @@ ROUTES = [("f32", "nn", 1, 32768, 255, "gemv"),  # 3.5
           ("f16", "nt", 2, 11008, 4096, "small"),  # 1.14 (rows)
           ("f16", "nt", 1, 16384, 2048, "small"),  # 1.3 (rows)
           ("f16", "nt", 1, 1024, 1024, "small"),  # 1.05 (rows)
+          ("f32", "nt", 2, 32768, 2048, "small"),  # 1.25 with W from HBM (rows)
           ("f16", "nt", 32, 32768, 512, "tiles"),  # 1.33 (rows)
           ("f32", "nt", 64, 11008, 256, "tiles"),  # 1.17 (rows)
           ("f32", "nn", 64, 16384, 512, "tiles"),  # 1.16 (rows)
