@@ -70,9 +70,10 @@ struct VecOf<float, 1> {
 // kernels have in NN: fp32 4 x 11008 x 4096 5.7e-7 against 2.9e-7 relative to float64, now 2.9e-7 in the
 // same time. FLUSH: with 17 to 32 rows there are no registers for that (28 spilled; two sums in AGPRs cost
 // 10-20%), and the sum of each round of loads is added to a total instead (with fewer rows, or in the
-// 8-wave shapes, that cost up to 20% where K is short).
+// 8-wave shapes, that cost up to 20% where K is short). fp32 sums of 4 waves need the two waves per SIMD: the
+// compiler then keeps them in VGPRs instead of copying them from AGPRs; fp16 loses 2-4% by it.
 template <typename T, bool TB, int FM, int FN, int KW, int D, int H, bool XV>
-__global__ void __launch_bounds__(KW * 64) __attribute__((amdgpu_waves_per_eu(KW > 8 ? KW / 4 : FM > 2 && KW == 4 ? 1 : 2)))
+__global__ void __launch_bounds__(KW * 64) __attribute__((amdgpu_waves_per_eu(KW > 4 ? KW / 4 : sizeof(T) == 4 && FM <= 2 ? 2 : 1)))
 gemm_rows_kernel(GemmParams p, int S) {
   typedef RowOps<T> Ops;
   typedef typename Ops::V V;
