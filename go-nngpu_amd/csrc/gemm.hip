@@ -1927,7 +1927,8 @@ int choose_split(int dtype, long M, long N, long K, bool beta, double *us = null
 
 // ------------------------------------------------------------------ fp32 on the bf16 cores
 // csrc/gemm_split.hip computes an fp32 product on the bf16 matrix cores at 1.6 times the speed of
-// the fp32 ones and with a smaller error. The dispatch prices both.
+// the fp32 ones and, for the sums of hundreds of terms that are priced here, with a smaller error.
+// The dispatch prices both.
 //
 // The price (us) of an fp32 product on the fp32 matrix cores: the tile model of choose_split, the
 // store of C, the packing of unaligned operands, and the second launch over K % 32.
@@ -2084,12 +2085,12 @@ bool takes_rows(const GemmDesc &d, const RowsPlan &rows, bool a_ok, bool b_ok, b
 
 // true when the product runs on the bf16 matrix cores: priced (the operands' packing, the
 // product, the reduce, 3 us for the fp32 kernels that stand behind it) at least 7% below the
-// fp32 matrix cores. Both prices were checked on 44 shapes (device times, fp32 -> bf16 parts, us):
-// taken 2048 x 2048 x 512 35 -> 35, 4096 x 4096 x 256 73 -> 60, 777 x 1234 x 4099 106 -> 74, 512 x
-// 11008 x 4096 369 -> 332, 2560^3 271 -> 167, 4096^3 928 -> 606; left on the fp32 cores, where the
-// packing or the fixed 15 us weigh too much: 1024^3 21 -> 35, 1280^3 42 -> 42, 256 x 4096 x 4096 71
-// -> 82, 128 x 8192 x 8192 139 -> 255. None of the 44 got slower; of those left, 512 x 4096 x 4096
-// would have gained most (125 -> 114).
+// fp32 matrix cores, or, with a raw B, below them. Both prices were checked on 44 shapes with packed
+// operands and 13 with a raw B (device times, fp32 -> bf16 parts, us): taken 2048 x 2048 x 512 35 -> 35,
+// 4096 x 4096 x 256 73 -> 60, 777 x 1234 x 4099 106 -> 74, 2560^3 271 -> 167, 4096^3 928 -> 606, raw 512 x
+// 11008 x 4096 367 -> 255, 256 x 4096 x 4096 72 -> 61 (W from HBM 92 -> 63); left on the fp32 cores, where
+// the packing or the fixed 15 us weigh too much: 1024^3 21 -> 35, 1280^3 42 -> 42, 128 x 8192 x 8192 139 ->
+// 255.
 bool cut_split(const GemmDesc &d, bool a_ok, bool b_ok, SplitCut *cut) {
   constexpr size_t kLimit = kScratchRetainBytes - 512;  // less the gate's block and the partials' rounding up
   long nb = d.batch, kc = d.K;

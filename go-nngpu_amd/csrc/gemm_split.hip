@@ -4,7 +4,10 @@
 // busy); the bf16 ones run at 16 times that rate. Every fp32 value v is the exact sum of three
 // bf16 values, h = bf16(v), m = bf16(v - h), l = v - h - m (round to nearest: 8 + 8 + 8 bits with
 // signs), and of the nine products of parts of a b six are computed in fp32 accumulators: hh, hm,
-// mh, mm, hl, lh. The others are at most 2^-24 |a b| together (2^-27 rms, of either sign). hh has
+// mh, mm, hl, lh (Henry, Tang and Heinecke, "Leveraging the bfloat16 artificial intelligence datatype
+// for higher-precision computations", ARITH 2019). The others are at most 2^-24 |a b| together (2^-27
+// rms, of either sign): a sum of one term is up to 1.67 2^-24 off where the fp32 cores round it to
+// 2^-24 (0.435 against 0.425 rms), sums of many come out closer. hh has
 // an accumulator of its own: the other five are 2^-8 of it and less, so a sum over K = 4096 rounds
 // at full size once per 32 k, where the fp32 cores do so every 4 k. Error against float64, N(0, 1)
 // operands, relative Frobenius: 4096^3 4.0e-7 against 1.15e-6 on the fp32 cores, 2048^3 2.7e-7
@@ -145,16 +148,16 @@ __device__ __forceinline__ void dma16s(const BufRsrc &s, unsigned voff, unsigned
 //    workgroup and K-tile); 144 KiB of LDS;
 //  * 128 x 128, 8 waves of 64 x 32: twice the tiles where those leave CUs idle (2048^3: 70 us
 //    against 109); three ring slots measured 1-2% slower than two.
-template <int BM, int BN, int WM, int WN, int BSRC, int RD, int WPE>
-__global__ void __launch_bounds__(WM * WN * 64) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
+template <int BM, int BN, int WM, int WN, int BSRC, int RD>
+__global__ void __launch_bounds__(WM * WN * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
 gemm_split_kernel(GemmParams p, SplitArgs q) {
   constexpr int NW = WM * WN, FM = BM / WM / 16, FN = BN / WN / 16, NS = 2;
   constexpr int CA = BM / 16 * 3, CB = BN / 16 * 3;  // 1 KiB chunks of a K-tile of A and of B
-  constexpr int IPA = (CA + NW - 1) / NW, IPB = BSRC ? 0 : CB / NW, LPW = IPA + IPB;
+  constexpr int IPA = CA / NW, IPB = BSRC ? 0 : CB / NW, LPW = IPA + IPB;
   static_assert(RD == 1 || RD == 2, "raw buffers");
   static_assert(BSRC == 0 || (BN == 128 && NW == 8), "a raw B: one 16-column block, or 64 columns x 8 k, per wave");
   constexpr int SLOT = (CA + CB) * 1024;
-  static_assert((CA % NW == 0 || CA < 2 * NW) && CB % NW == 0, "tile shape");
+  static_assert(CA % NW == 0 && CB % NW == 0, "tile shape");
   static_assert(WM * 16 * (BN + 4) * 4 <= NS * SLOT, "epilogue staging exceeds the ring");
   __shared__ __attribute__((aligned(1024))) char smem[NS * SLOT];
   if (split_product_skipped(*p.gate, p.gate_seq)) return;  // uniform: no workgroup of this launch writes that word
@@ -173,8 +176,7 @@ gemm_split_kernel(GemmParams p, SplitArgs q) {
   unsigned soa[IPA], sob[IPB ? IPB : 1];
 #pragma unroll
   for (int i = 0; i < IPA; ++i) {
-    // (with 12 chunks for 8 waves the last ones copy chunk 11 again)
-    const int c = min(wave * IPA + i, CA - 1), blk = min((int)(m0 >> 4) + c / 3, q.nra - 1);
+    const int c = wave * IPA + i, blk = min((int)(m0 >> 4) + c / 3, q.nra - 1);
     soa[i] = (unsigned)blk * (unsigned)q.nkt * kSplitBlock + (unsigned)kt0 * kSplitBlock + (c % 3) * 1024;
   }
 #pragma unroll
@@ -189,7 +191,7 @@ gemm_split_kernel(GemmParams p, SplitArgs q) {
     for (int i = 0; i < IPA; ++i)
       if (2 * i / LPW == h)
         dma16s(ra, voff, __builtin_amdgcn_readfirstlane(soa[i] + ko),
-               __builtin_amdgcn_readfirstlane(st + min(wave * IPA + i, CA - 1) * 1024));
+               __builtin_amdgcn_readfirstlane(st + (wave * IPA + i) * 1024));
 #pragma unroll
     for (int i = 0; i < IPB; ++i)
       if (2 * (IPA + i) / LPW == h)
@@ -350,12 +352,12 @@ gemm_split_kernel(GemmParams p, SplitArgs q) {
   store_tile_rows<BM, BN, WM, WN>(p, m0, n0, z, reinterpret_cast<float *>(smem), acc);
 }
 
-template <int BM, int BN, int WM, int WN, int BSRC = 0, int RD = 1, int WPE = 2>
+template <int BM, int BN, int WM, int WN, int BSRC = 0, int RD = 1>
 hipError_t launch_tile(GemmParams p, const SplitArgs &q, long batch, hipStream_t s) {
   p.tiles_m = (int)((p.M + BM - 1) / BM);
   p.tiles_n = (int)((p.N + BN - 1) / BN);
   const dim3 grid((unsigned)(p.tiles_m * p.tiles_n), 1, (unsigned)(batch * q.S));
-  hipLaunchKernelGGL((gemm_split_kernel<BM, BN, WM, WN, BSRC, RD, WPE>), grid, dim3(WM * WN * 64), 0, s, p, q);
+  hipLaunchKernelGGL((gemm_split_kernel<BM, BN, WM, WN, BSRC, RD>), grid, dim3(WM * WN * 64), 0, s, p, q);
   return hipGetLastError();
 }
 

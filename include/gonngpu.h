@@ -312,8 +312,10 @@ int gn_synchronize(void *stream, CError *err);
  *   C[M,N] = act( alpha * op(A) * op(B) + beta * C + bias[n] )
  * op(A) is A[M,K] (lda >= K) or, with transA, A stored [K,M] (lda >= M); likewise B.
  * dtype GN_F32: A, B fp32, on v_mfma_f32_16x16x4_f32 or, for large products, as exact sums of
- * three bf16 parts on the bf16 MFMA with fp32 accumulation (no larger error; operands with
- * infinities, NaN or magnitudes of 2^36 and above take the fp32 MFMA).
+ * three bf16 parts on the bf16 MFMA with fp32 accumulation (sums come out closer than on the fp32
+ * MFMA; a sum of one term may be 1.67 2^-24 off where the fp32 MFMA rounds it to 2^-24; operands
+ * with infinities, NaN or magnitudes of 2^36 and above take the fp32 MFMA, after the time of the
+ * pack or, for at most some 500 rows, of the product).
  * dtype GN_F16: A, B fp16, fp32 accumulate (v_mfma_f32_16x16x32_f16).
  * C and bias are fp32; bias may be NULL; beta == 0 never reads C.
  * batch >= 1 with element strides strideA/B/C between consecutive problems.

@@ -739,7 +739,7 @@ def test_skinny_linear_layer_all_layouts(dev, dtype, M, N, K):
                                          (G.GN_F16, 2, 8200, 1024), (G.GN_F16, 4, 16384, 515)])
 def test_gemv_nn_rows_all_layouts(dev, dtype, M, N, K):
     """Products of 1-4 rows with W stored K x N (NN, the reference LinearLayer's input @ Weight)
-    run on the GEMV kernel (K split over 16 waves, fp32 sums on the VALU). NaN start; bias +
+    run on the few-rows or the GEMV kernel (K split over the waves of a workgroup). NaN start; bias +
     GELU, then alpha / beta with a prior C, each against float64 of the stored operands (relFrob
     1e-5); the same product in the other layouts (other kernels, other summation orders) within
     the same bar; and two runs bit for bit."""

@@ -13,7 +13,7 @@ reference's formulas) applied to the float64 pre-activation. The padding columns
 left as they were.
 
 The second: 120 products of 1-16 rows with wide N and long K (test_gemm_random_few_rows),
-where the dispatch chooses between the GEMV, small-product and tiled kernels."""
+where the dispatch chooses between the few-rows, GEMV, small-product and tiled kernels."""
 import random
 import sys
 
@@ -100,8 +100,8 @@ def test_gemm_random_sweep(dev, seed):
 def test_gemm_random_few_rows(dev, seed):
     """120 products of 1-16 rows with wide N (256 .. 20000) and long K (1 .. 9000), drawn over
     dtypes, all four layouts, padded leading dimensions, alpha, beta with a prior C, bias and
-    ReLU / GELU: the range where the dispatch chooses between the NN GEMV kernel, the
-    small-product kernel (its skinny linear-layer branch included) and the tiled kernels. Each
+    ReLU / GELU: the range where the dispatch chooses between the few-rows kernel (csrc/gemm_rows.hip), the
+    NN GEMV kernel, the small-product kernel (its skinny linear-layer branch included) and the tiled kernels. Each
     against float64 of the stored operands (relFrob <= 1e-5; GELU through the oracle's
     formula), C's padding columns untouched."""
     import torch

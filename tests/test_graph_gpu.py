@@ -1,5 +1,6 @@
 """HIP graph capture of the device-pointer API: the GEMM (fp16 ring and register-staged
-kernels, fp32, the small-product kernel in fp32 and for a skinny fp16 X W^T, the NN GEMV), CSR SpMM, SpMV and the grouped-layout SpMV of a plan built before the capture
+kernels, fp32, the small-product kernel in fp32 and for a skinny unaligned fp16 X W^T, the few-rows
+kernel in both layouts, the NN GEMV), CSR SpMM, SpMV and the grouped-layout SpMV of a plan built before the capture
 launch no memset and allocate nothing, so a caller can capture them once and replay the graph. Each replay is compared with the eager result
 for inputs changed between replays (with the program's own eager work and
 synchronisations in between), bit for bit."""
@@ -28,10 +29,14 @@ def test_graph_replays_match_eager(dev):
     x32 = torch.randn(700, 300, device=dev)              # fp32 register-staged kernel
     xs = torch.randn(96, 200, device=dev)                # fp32 small-product kernel
     ws = torch.randn(200, 80, device=dev)
-    xk = torch.randn(2, 4096, device=dev).half()         # fp16 skinny X W^T: small-product kernel
+    xk = torch.randn(2, 4096, device=dev).half()         # fp16 X W^T of two rows: few-rows kernel
     wk = (0.05 * torch.randn(2048, 4096, device=dev)).half()
-    xg = torch.randn(1, 2048, device=dev)                 # fp32 NN GEMV (one row)
+    xg = torch.randn(1, 2048, device=dev)                 # fp32 X W of one row: few-rows kernel
     wg = 0.05 * torch.randn(2048, 8192, device=dev)
+    xu = torch.randn(2, 4090, device=dev).half()          # fp16 X W^T, rows off 16 bytes: small-product kernel
+    wu = (0.05 * torch.randn(2048, 4090, device=dev)).half()
+    xv1 = torch.randn(1, 128, device=dev)                 # fp32 X W with little K: GEMV
+    wv1 = 0.05 * torch.randn(128, 8192, device=dev)
     w32 = torch.randn(300, 500, device=dev)
     bias = torch.randn(500, device=dev)
     a2 = torch.randn(4600, 64, device=dev).half()        # fp16 row split: two launches
@@ -47,6 +52,8 @@ def test_graph_replays_match_eager(dev):
     ys = torch.empty(96, 80, device=dev)
     yk = torch.empty(2, 2048, device=dev)
     yg = torch.empty(1, 8192, device=dev)
+    yu = torch.empty(2, 2048, device=dev)
+    yv1 = torch.empty(1, 8192, device=dev)
     S = torch.empty(4000, 64, device=dev)
     yv = torch.empty(4000, device=dev)
     yp = torch.empty(4000, device=dev)
@@ -60,6 +67,8 @@ def test_graph_replays_match_eager(dev):
         G.gemm(xs, ws, ys, bias=bias[:80], act=G.ACT_RELU)
         G.gemm(xk, wk, yk, transB=True)
         G.gemm(xg, wg, yg, bias=bias.repeat(17)[:8192], act=G.ACT_RELU)
+        G.gemm(xu, wu, yu, transB=True)
+        G.gemm(xv1, wv1, yv1)
         G.spmm_csr(4000, 64, 3000, val.size, d_rp, d_col, d_val, D, S)
         G.spmv_csr(4000, 3000, val.size, d_rp, d_col, d_val, xv, yv)
         plan.run(d_val, xv, yp)
@@ -76,7 +85,7 @@ def test_graph_replays_match_eager(dev):
     torch.cuda.synchronize()
 
     assert val.size >= 1 << 16
-    outs = (c16, c2, y32, S, yv, yp, ys, yk, yg)
+    outs = (c16, c2, y32, S, yv, yp, ys, yk, yg, yu, yv1)
     for rep in range(3):
         # new inputs, eager work and a synchronisation between replays
         with torch.no_grad():
@@ -86,6 +95,8 @@ def test_graph_replays_match_eager(dev):
             ws.mul_(-0.5).add_(0.2)
             xk.copy_(torch.randn_like(xk, dtype=torch.float32).half())
             xg.mul_(-1.25)
+            xu.copy_(torch.randn_like(xu, dtype=torch.float32).half())
+            xv1.mul_(-0.75)
             D.copy_(torch.randn_like(D))
             xv.mul_(-1.5)
             d_val.mul_(0.75)
@@ -96,7 +107,7 @@ def test_graph_replays_match_eager(dev):
         work()  # eager, on the current stream
         torch.cuda.synchronize()
         for name, gt, ref in zip(("gemm f16", "gemm f16 row split", "gemm f32", "spmm", "spmv", "spmv plan",
-                                  "gemm f32 small", "gemm f16 skinny", "gemv f32"), got,
+                                  "gemm f32 small", "rows f16", "rows f32", "gemm f16 skinny", "gemv f32"), got,
                                  outs):
             same = torch.equal(gt, ref)
             _say("replay", rep, name, "bit-identical" if same else "DIFFERS")
