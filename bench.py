@@ -32,8 +32,8 @@ operands with the headline's distributions and on all-zero operands. Under the b
 power limit the clock, and so this rate, depends on the operand values; the first figure
 is the most any GEMM on such data can reach on the box.
 
-`rows` times products of a few rows (a linear layer at batch 1-16 on the row-streaming
-kernels, a small MLP layer) beside torch.mm, for scale.
+`rows` times products of a few rows (a linear layer at batch 1-16, a small MLP layer) beside
+torch.mm, for scale.
 
 `--only a,b,...` runs a subset of {c3, ceiling, c2, c1, c4, rows, spmm, spmv, e2e, copy} (used by
 the rocprofv3 passes that produce profiles/); `copy` is a 1 GiB device copy used to
@@ -469,7 +469,7 @@ def run_c4(c, steps, warmup):
 def run_rows(c, steps):
     """Products of a few rows beside torch.mm (TF32 off; fp32 output for fp16 inputs), event
     timing of back-to-back launches: X W with W stored K x N (NN), X W^T with W
-    stored N x K (NT), both on the row-streaming kernels, and a small MLP layer. The rate
+    stored N x K (NT), and a small MLP layer. The rate
     is W's bytes over the time (W is read once; X and C are a few rows)."""
     t = c.torch
     t.backends.cuda.matmul.allow_tf32 = False

@@ -25,7 +25,7 @@
 //
 // us on MI355X, W from HBM (before -> after): fp32 NT 16 x 11008 x 4096 59 -> 44, 16 x 5000 x 800 21 -> 9,
 // 16 x 1024 x 4096 19.6 -> 11, 8 x 3000 x 2000 49 -> 10, 32 x 11008 x 4096 75 -> 53; NN 16 x 11008 x 4096
-// 64 -> 41, 1 x 4096 x 4096 30 -> 20; fp16 NT 16 x 4096 x 1024 11.8 -> 5.5, NN 4 x 11008 x 4096 27 -> 21, 1 x
+// 64 -> 41, 1 x 4096 x 4096 30 -> 20; fp16 NT 16 x 4096 x 1024 11.8 -> 5.5, NN 4 x 11008 x 4096 25 -> 20, 1 x
 // 2048 x 8192 45 -> 14.
 #include <algorithm>
 

@@ -19,9 +19,9 @@
 // x 2^16 y 2^16 overflows). The pack kernel looks, and the product kernel in a B that it splits itself;
 // otherwise, infinities and NaN included, the fp32 kernels enqueued behind them compute C (split_gate.h).
 //
-// Time, 4096^3 NN: pack 62-75 us (335 MB at copy rate), product 508 us = 270 TFLOP/s, 1.62 PFLOP/s of
-// bf16 products, which is the rate the board's power limit leaves the matrix cores; 928 -> 606 us
-// in all.
+// Time, 4096^3 NN: 928 -> 605-620 us a call, 56 of them the pack (335 MB, 6 TB/s), about 5 the fp32 kernels
+// that return at once; the product's 545-560 are 245-250 TFLOP/s, 1.5 PFLOP/s of bf16 products, which is the
+// rate the board's power limit leaves the matrix cores.
 #include <algorithm>
 
 #include "gemm_split.h"
