@@ -394,12 +394,17 @@ bool plan_split(const GemmDesc &d, long nb, long kc, SplitPlan *out) {
   // 1024: level). It reads 16-byte vectors of a K-contiguous B, in every batch and part (kc is a
   // multiple of 32, or K).
   const bool raw_ok = d.tb ? vectors(d.B, d.ldb, d.strideB, d.batch) && d.K % 4 == 0 : true;
+  // A K-contiguous operand off 16 bytes is packed element by element: past what the caches hold its packing
+  // takes 1.6 times as long (17 x 130 x 2567 x 2071 TT 594 us where 411 were priced and the fp32 cores take 466).
+  const bool odd_a = !d.ta && !vectors(d.A, d.lda, d.strideA, d.batch), odd_b = d.tb && !vectors(d.B, d.ldb, d.strideB, d.batch);
   out->us = 1e30;
   for (int form = 0; form < 4; ++form) {
     const int tile = form & 1;
     const bool raw = form >= 2;
     if (raw ? !raw_ok : pb >= ring::kNumRecords) continue;
-    const double pack_us = 3.0 + (double)batch * (double)(M + (raw ? 0 : N)) * (double)K * 10.0 / 4.6e6;
+    const double packed_mb = 6.0e-6 * (double)batch * (double)(M + (raw ? 0 : N)) * (double)K;
+    const double a_bytes = odd_a && packed_mb > 100.0 ? 16.0 : 10.0, b_bytes = odd_b && packed_mb > 100.0 ? 16.0 : 10.0;
+    const double pack_us = 3.0 + (double)batch * (a_bytes * (double)M + (raw ? 0.0 : b_bytes * (double)N)) * (double)K / 4.6e6;
     const double w_us = raw ? (double)batch * (double)N * (double)K * 4.0 / 4.9e6 : 0.0;
     const long bm = tile == 0 ? 256 : 128;
     const long tiles = ((M + bm - 1) / bm) * ((N + 127) / 128) * batch;

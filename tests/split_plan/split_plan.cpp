@@ -39,12 +39,16 @@ struct Seen {
   long cuts = 0, raw = 0, raw_in_batch = 0, batch_cut = 0, one_batch = 0, k_cut = 0, raw_k_cut = 0, odd_stride = 0;
 } g_seen;
 
-void check(const GemmDesc &d) {
-  SplitCut c;
+bool cut(const GemmDesc &d, SplitCut *c) {
   const bool a_ok = d.lda % 4 == 0 && (d.batch == 1 || d.strideA % 4 == 0) && (d.ta ? d.M : d.K) % 4 == 0;
   const bool b_ok = (uintptr_t)d.B % 16 == 0 && d.ldb % 4 == 0 && (d.batch == 1 || d.strideB % 4 == 0) &&
                     (d.tb ? d.K : d.N) % 4 == 0;
-  if (!cut_split(d, a_ok, b_ok, &c)) return;
+  return cut_split(d, a_ok, b_ok, c);
+}
+
+void check(const GemmDesc &d) {
+  SplitCut c;
+  if (!cut(d, &c)) return;
   ++g_seen.cuts;
   g_seen.raw += c.plan.raw_b;
   g_seen.raw_in_batch += c.plan.raw_b && d.batch > 1;
@@ -119,7 +123,7 @@ int main(int argc, char **argv) {
     const GemmDesc d = product(std::atol(argv[1]), std::atol(argv[2]), std::atol(argv[3]), std::atol(argv[4]),
                                argv[5][0] == 't', argv[5][1] == 't', std::atol(argv[6]));
     SplitCut c;
-    if (cut_split(d, true, d.strideB % 4 == 0, &c))
+    if (cut(d, &c))
       std::printf("nb %ld kc %ld raw %d S %d\n", c.nb, c.kc, (int)c.plan.raw_b, c.plan.S);
     else
       std::printf("none\n");
