@@ -254,8 +254,9 @@ def _current_stream():
     that is not part of torch's public interface: without it, the Stream object is built."""
     import torch
 
-    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
-    if raw is None:
+    try:
+        raw = torch._C._cuda_getCurrentRawStream
+    except AttributeError:
         return torch.cuda.current_stream().cuda_stream
     return raw(torch.cuda.current_device())
 
